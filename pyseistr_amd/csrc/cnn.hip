@@ -609,147 +609,290 @@ conv32z(const __bf16 *__restrict__ in, const __bf16 *__restrict__ Wg, const floa
 
 // ---------------------------------------------------------------------------
 // Weight gradient of a 32-channel layer: dW[t][ci][co] = sum_v in[v+t][ci]
-// g[v][co] over the voxels of each block (64 (i1) x 4 (i2) at one i3), on
-// the matrix cores with K = voxels.  The block stages its input tile with
-// halo ([ci][voxel] transposed) and the output gradient ([co][voxel]) in
-// LDS; wave w accumulates taps t = w, w+4, ... and writes its partial
-// [27][32][32] sums to part[block]; db partials go to pb[block][32].
+// g[v][co], on the matrix cores with K = voxels.
+//
+// Both operands have K along the slow axis of the channels-last layout, so
+// the tiles are staged as they lie ([voxel][32], 16-byte copies) and the
+// fragments come out of LDS through the transposing read
+// (ds_read_b64_tr_b16): a tap's shift is then a whole-voxel offset and every
+// read stays aligned.  A block walks tiles of 64 (i1) x 4 (i2) voxels along
+// i3 and keeps its sums in registers: wave (d2, kh) holds the nine taps of
+// one i2 shift (144 accumulators) for the rows of one half of the tile, so
+// at most WG_BLOCKS partials are written and reduced, whatever the volume.
+// For dilation 1 the three input planes are a ring in LDS and the next
+// plane and gradient tile are loaded into registers while the current one is
+// multiplied; larger dilations stage one plane at a time.
+// 64^3, one layer: 144 us (2-byte staging, eight 2-byte LDS reads per
+// fragment, 1024 partials) + 238 us (their serial sum) before.
 // ---------------------------------------------------------------------------
-constexpr int WG_X = 64, WG_Y = 4;
+constexpr int WG_X = 64, WG_Y = 4, WG_TB = 384, WG_BLOCKS = 256;
 constexpr int MAX_DIL = 8;
-constexpr int WG_HXM = WG_X + 2 * MAX_DIL, WG_HYM = WG_Y + 2 * MAX_DIL;
+constexpr int WG_PART = NT * C * C + C;  // one block's partial: weights, then bias
+constexpr int WG_GCH = WG_X * WG_Y * 4;  // 16-byte chunks of a gradient tile
 
-// The input is staged one tap plane (d3) at a time, with an in-plane halo
-// of `dil` voxels; the 9 taps of a plane are split over the 4 waves.
-__global__ void __launch_bounds__(TB)
-conv32_wgrad(const __bf16 *__restrict__ in, const __bf16 *__restrict__ g, float *__restrict__ part,
-             float *__restrict__ pb, int n1, int n2, int n3, int dil) {
-    // input plane [ci][y HY][x HX], gradient tile [co][y][x]
-    __shared__ __bf16 ti[C * WG_HYM * WG_HXM];
-    __shared__ __bf16 tg[C * WG_Y * WG_X];
-    const int HX = WG_X + 2 * dil, HY = WG_Y + 2 * dil;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int ntx = (n1 + WG_X - 1) / WG_X, nty = (n2 + WG_Y - 1) / WG_Y;
-    long bid = blockIdx.x;
-    const int x0 = (int)(bid % ntx) * WG_X;
-    bid /= ntx;
-    const int y0 = (int)(bid % nty) * WG_Y;
-    const int z = (int)(bid / nty);
-    const long n12 = (long)n1 * n2;
-    for (int i = threadIdx.x; i < WG_Y * WG_X; i += blockDim.x) {
-        int xx = i % WG_X, yy = i / WG_X;
-        int j1 = x0 + xx, j2 = y0 + yy;
-        bool ok = j1 < n1 && j2 < n2;
-        const __bf16 *src = g + ((long)j1 + (long)j2 * n1 + (long)z * n12) * C;
-        for (int c = 0; c < C; c++) tg[c * (WG_Y * WG_X) + i] = ok ? src[c] : (__bf16)0.0f;
-    }
-    const int kq = (lane >> 5) * 8;
-    for (int zz = 0; zz < 3; zz++) {
-        const int j3 = z + (zz - 1) * dil;
-        __syncthreads();  // the previous plane's readers are done
-        for (int i = threadIdx.x; i < HY * HX; i += blockDim.x) {
-            int xx = i % HX, yy = i / HX;
-            int j1 = x0 - dil + xx, j2 = y0 - dil + yy;
-            bool ok = j1 >= 0 && j1 < n1 && j2 >= 0 && j2 < n2 && j3 >= 0 && j3 < n3;
-            const __bf16 *src = in + ((long)j1 + (long)j2 * n1 + (long)j3 * n12) * C;
-            for (int c = 0; c < C; c++) ti[c * (HY * HX) + i] = ok ? src[c] : (__bf16)0.0f;
-        }
-        __syncthreads();
-        for (int tt = w; tt < 9; tt += 4) {
-            const int t = zz * 9 + tt;
-            const int d1 = (tt % 3 - 1) * dil, d2 = (tt / 3 - 1) * dil;
-            f32x16 acc;
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-            // K = voxels, 16 per MFMA: rows yy, x chunks of 16
-            for (int yy = 0; yy < WG_Y; yy++) {
-                for (int xc = 0; xc < WG_X; xc += 16) {
-                    // A[row = ci][k = voxel]: lane -> ci = lane & 31, voxels xc + kq .. +7
-                    bf16x8 a, b;
-                    const __bf16 *ai = ti + (lane & 31) * (HY * HX) + (yy + d2 + dil) * HX + (xc + kq + d1 + dil);
-                    const __bf16 *bg = tg + (lane & 31) * (WG_Y * WG_X) + yy * WG_X + xc + kq;
-#pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        a[i] = ai[i];
-                        b[i] = bg[i];
-                    }
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-                }
-            }
-            // D[row = ci][col = co]
-            float *dst = part + (size_t)blockIdx.x * NT * C * C + (size_t)t * C * C;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                int ci = (r / 4) * 8 + (lane >> 5) * 4 + (r % 4);
-                dst[ci * C + (lane & 31)] = acc[r];
-            }
-        }
-    }
-    // bias partials: sum of g over the tile per channel
-    if (threadIdx.x < C) {
-        float s = 0.0f;
-        for (int i = 0; i < WG_Y * WG_X; i++) s += (float)tg[threadIdx.x * (WG_Y * WG_X) + i];
-        pb[(size_t)blockIdx.x * C + threadIdx.x] = s;
-    }
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+
+// The 32 x 16 fragment (row = channel, k = voxel) of 16 consecutive voxels
+// starting at p, p = [voxel][32] in LDS: lane l gets channel l & 31, voxels
+// (l >> 5) * 8 + 0..7.  In each group of 16 lanes lane i supplies the 8 bytes
+// of voxel i / 4, channels 4 (i % 4) .. +3, and receives channel i of the
+// group's four voxels.  off = tr_off(lane), in elements.
+__device__ inline int tr_off(int lane) {
+    const int g = lane >> 4, i = lane & 15;
+    return ((g >> 1) * 8 + (i >> 2)) * C + (g & 1) * 16 + (i & 3) * 4;
+}
+__device__ inline bf16x8 tr_frag(const __bf16 *p, int off) {
+    const i16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(p + off));
+    const i16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(p + off + 4 * C));
+    const bf16x4 x = __builtin_bit_cast(bf16x4, a), y = __builtin_bit_cast(bf16x4, b);
+    return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// Layer 1 weight gradient: dW1[t][co] = sum_v x[v+t] g1[v][co]; block
-// partials over 256 voxels; thread (t, co) pairs.
-__global__ void __launch_bounds__(1024)
-conv1_wgrad(const float *__restrict__ x, float xscale, const __bf16 *__restrict__ g, float *__restrict__ part, int n1,
-            int n2, int n3, int vox_per_block, int dil) {
-    long n = (long)n1 * n2 * n3;
-    long v0 = (long)blockIdx.x * vox_per_block;
-    int tid = threadIdx.x;
-    float s = 0.0f, sb = 0.0f;
-    int t = tid / C, co = tid % C;
-    if (tid < NT * C) {
-        int d1 = (t % 3 - 1) * dil, d2 = ((t / 3) % 3 - 1) * dil, d3 = (t / 9 - 1) * dil;
-        for (long v = v0; v < std::min(n, v0 + vox_per_block); v++) {
-            int i1 = (int)(v % n1);
-            long r = v / n1;
-            int i2 = (int)(r % n2), i3 = (int)(r / n2);
-            int j1 = i1 + d1, j2 = i2 + d2, j3 = i3 + d3;
-            bool ok = j1 >= 0 && j1 < n1 && j2 >= 0 && j2 < n2 && j3 >= 0 && j3 < n3;
-            float gv = (float)g[v * C + co];
-            if (ok) s += (x[v + d1 + (long)n1 * (d2 + (long)n2 * d3)] * xscale) * gv;
-            if (t == 0) sb += gv;
+template <bool RING>
+__global__ void __launch_bounds__(WG_TB)
+conv32_wgrad(const __bf16 *__restrict__ in, const __bf16 *__restrict__ g, float *__restrict__ part, int n1, int n2,
+             int n3, int dil) {
+    constexpr int RPL = (WG_X + 2) * (WG_Y + 2);  // voxels of a plane of the ring
+    constexpr int NP = RING ? (RPL * 4 + WG_TB - 1) / WG_TB : 1, NG = (WG_GCH + WG_TB - 1) / WG_TB;
+    __shared__ uint4 wg_lds[WG_GCH + (RING ? 3 * RPL : (WG_X + 2 * MAX_DIL) * (WG_Y + 2 * MAX_DIL)) * 4];
+    const int HX = WG_X + 2 * dil, HY = WG_Y + 2 * dil, pl = HX * HY;
+    uint4 *const gt = wg_lds, *const it = wg_lds + WG_GCH;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int d2 = w % 3, kh = w / 3;
+    const int ntx = (n1 + WG_X - 1) / WG_X, nty = (n2 + WG_Y - 1) / WG_Y;
+    const long n12 = (long)n1 * n2, ntiles = (long)ntx * nty * n3;
+    const long per = (ntiles + gridDim.x - 1) / gridDim.x;
+    long item = (long)blockIdx.x * per;
+    const long end = min(ntiles, item + per);
+    const int toff = tr_off(lane);
+    const uint4 zero = {0u, 0u, 0u, 0u};
+    f32x16 acc[9];
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+    float bias = 0.0f;
+    int x0 = 0, y0 = 0;
+    // 16-byte chunk c of the input plane j3 / of the gradient tile at z
+    auto in_chunk = [&](int c, int j3) -> uint4 {
+        const int v = c >> 2, xx = v % HX, yy = v / HX;
+        const int j1 = x0 - dil + xx, j2 = y0 - dil + yy;
+        if (j1 < 0 || j1 >= n1 || j2 < 0 || j2 >= n2 || j3 < 0 || j3 >= n3) return zero;
+        return reinterpret_cast<const uint4 *>(in)[((long)j1 + (long)j2 * n1 + (long)j3 * n12) * 4 + (c & 3)];
+    };
+    auto g_chunk = [&](int c, int z) -> uint4 {
+        const int v = c >> 2, j1 = x0 + (v & (WG_X - 1)), j2 = y0 + v / WG_X;
+        if (j1 >= n1 || j2 >= n2 || z >= n3) return zero;
+        return reinterpret_cast<const uint4 *>(g)[((long)j1 + (long)j2 * n1 + (long)z * n12) * 4 + (c & 3)];
+    };
+    // the taps (d3 = zz - 1, this wave's d2) of the tile, its input plane at ip
+    auto taps = [&](int zz, const __bf16 *ip) {
+        const __bf16 *gp = reinterpret_cast<const __bf16 *>(gt);
+#pragma unroll 1
+        for (int yy = 2 * kh; yy < 2 * kh + 2; yy++)
+#pragma unroll 2
+            for (int xc = 0; xc < WG_X; xc += 16) {
+                const bf16x8 b = tr_frag(gp + (yy * WG_X + xc) * C, toff);
+                if (zz == 1 && d2 == 0) {
+#pragma unroll
+                    for (int i = 0; i < 8; i++) bias += (float)b[i];
+                }
+#pragma unroll
+                for (int d1 = 0; d1 < 3; d1++) {
+                    const bf16x8 a = tr_frag(ip + ((yy + d2 * dil) * HX + xc + d1 * dil) * C, toff);
+                    if (zz == 0) acc[d1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[d1], 0, 0, 0);
+                    else if (zz == 1) acc[3 + d1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[3 + d1], 0, 0, 0);
+                    else acc[6 + d1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[6 + d1], 0, 0, 0);
+                }
+            }
+    };
+    while (item < end) {
+        const long col = item / n3;
+        const int za = (int)(item % n3), zb = (int)min<long>((long)n3, za + (end - item));
+        item += zb - za;
+        x0 = (int)(col % ntx) * WG_X;
+        y0 = (int)(col / ntx) * WG_Y;
+        if constexpr (RING) {
+            __syncthreads();  // the previous column's readers are done
+            for (int c = threadIdx.x; c < pl * 4; c += WG_TB) {
+                it[((za + 2) % 3) * (RPL * 4) + c] = in_chunk(c, za - 1);
+                it[(za % 3) * (RPL * 4) + c] = in_chunk(c, za);
+            }
+            uint4 pi[NP], pg[NG];
+            auto fetch = [&](int z) {  // what tile z needs that is not in LDS yet
+#pragma unroll
+                for (int k = 0; k < NP; k++) {
+                    const int c = threadIdx.x + k * WG_TB;
+                    pi[k] = c < RPL * 4 ? in_chunk(c, z + 1) : zero;
+                }
+#pragma unroll
+                for (int k = 0; k < NG; k++) {
+                    const int c = threadIdx.x + k * WG_TB;
+                    pg[k] = c < WG_GCH ? g_chunk(c, z) : zero;
+                }
+            };
+            fetch(za);
+#pragma unroll 1
+            for (int z = za; z < zb; z++) {
+                if (z > za) __syncthreads();
+#pragma unroll
+                for (int k = 0; k < NP; k++) {
+                    const int c = threadIdx.x + k * WG_TB;
+                    if (c < RPL * 4) it[((z + 1) % 3) * (RPL * 4) + c] = pi[k];
+                }
+#pragma unroll
+                for (int k = 0; k < NG; k++) {
+                    const int c = threadIdx.x + k * WG_TB;
+                    if (c < WG_GCH) gt[c] = pg[k];
+                }
+                __syncthreads();
+                if (z + 1 < zb) fetch(z + 1);
+                const __bf16 *ip = reinterpret_cast<const __bf16 *>(it);
+                taps(0, ip + ((z + 2) % 3) * (RPL * C));
+                taps(1, ip + (z % 3) * (RPL * C));
+                taps(2, ip + ((z + 1) % 3) * (RPL * C));
+            }
+        } else {
+#pragma unroll 1
+            for (int z = za; z < zb; z++) {
+                auto plane = [&](int zz) {
+                    __syncthreads();
+                    if (zz == 0)
+                        for (int c = threadIdx.x; c < WG_GCH; c += WG_TB) gt[c] = g_chunk(c, z);
+                    for (int c = threadIdx.x; c < pl * 4; c += WG_TB) it[c] = in_chunk(c, z + (zz - 1) * dil);
+                    __syncthreads();
+                };
+                plane(0);
+                taps(0, reinterpret_cast<const __bf16 *>(it));
+                plane(1);
+                taps(1, reinterpret_cast<const __bf16 *>(it));
+                plane(2);
+                taps(2, reinterpret_cast<const __bf16 *>(it));
+            }
         }
-        part[(size_t)blockIdx.x * (NT * C + C) + tid] = s;
-        if (t == 0) part[(size_t)blockIdx.x * (NT * C + C) + NT * C + co] = sb;
     }
+    // the two halves' sums meet in LDS, three taps at a time (3 waves x 48 x
+    // 64 floats = 36 KB, within the staging area)
+    float *const sh = reinterpret_cast<float *>(wg_lds);
+    float *const dst = part + (size_t)blockIdx.x * WG_PART;
+    bias += __shfl_xor(bias, 32);  // the lane pair of a channel
+    auto meet = [&](int zz, const f32x16 *a) {
+        __syncthreads();
+        if (kh == 1)
+#pragma unroll
+            for (int d1 = 0; d1 < 3; d1++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) sh[(d2 * 48 + d1 * 16 + r) * 64 + lane] = a[d1][r];
+        __syncthreads();
+        if (kh == 0)
+#pragma unroll
+            for (int d1 = 0; d1 < 3; d1++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {  // D[row = ci][col = co]
+                    const int ci = (r / 4) * 8 + (lane >> 5) * 4 + (r % 4), t = zz * 9 + d2 * 3 + d1;
+                    dst[(t * C + ci) * C + (lane & 31)] = a[d1][r] + sh[(d2 * 48 + d1 * 16 + r) * 64 + lane];
+                }
+    };
+    meet(0, acc);
+    meet(1, acc + 3);
+    meet(2, acc + 6);
+    __syncthreads();
+    if (d2 == 0 && kh == 1 && lane < C) sh[lane] = bias;
+    __syncthreads();
+    if (d2 == 0 && kh == 0 && lane < C) dst[NT * C * C + lane] = bias + sh[lane];
+}
+
+// Layer 1 weight gradient: dW1[t][co] = sum_v x[v+t] g1[v][co] in FP32 on the
+// matrix cores (v_mfma_f32_32x32x2_f32): rows are the 27 taps and a row of
+// ones for the bias, k = two voxels of a trace, columns the channels.  One
+// wave takes whole traces, so the tests of a tap's i2 and i3 shift are made
+// once a trace and its loads run along i1.  64^3: 408 us as one thread per
+// (tap, channel) walking 256 voxels, before.
+constexpr int C1_BLOCKS = 512;
+constexpr int C1_PART = (NT + 1) * C;
+__global__ void __launch_bounds__(TB)
+conv1_wgrad(const float *__restrict__ x, float xscale, const __bf16 *__restrict__ g, float *__restrict__ part, int n1,
+            int n2, int n3, int dil) {
+    __shared__ float sh[4][C * C];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, t = lane & 31, hi = lane >> 5, co = t;
+    const int d1 = (t % 3 - 1) * dil, d2 = ((t / 3) % 3 - 1) * dil, d3 = (t / 9 - 1) * dil;
+    const long rows = (long)n2 * n3;
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+    for (long row = (long)blockIdx.x * 4 + w; row < rows; row += (long)gridDim.x * 4) {
+        const int i2 = (int)(row % n2), i3 = (int)(row / n2), j2 = i2 + d2, j3 = i3 + d3;
+        const bool ok = t < NT && j2 >= 0 && j2 < n2 && j3 >= 0 && j3 < n3;
+        const float *xr = x + (ok ? ((long)j3 * n2 + j2) * n1 : 0);
+        const __bf16 *gr = g + row * n1 * C + co;
+        for (int v0 = 0; v0 < n1; v0 += 16) {
+            float a[8], b[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const int i1 = v0 + 2 * k + hi, j1 = i1 + d1;
+                const bool in1 = i1 < n1, tap = ok && in1 && j1 >= 0 && j1 < n1;
+                const float gv = (float)gr[(long)(in1 ? i1 : 0) * C], xv = xr[tap ? j1 : 0] * xscale;
+                a[k] = tap ? xv : (t == NT ? 1.0f : 0.0f);
+                b[k] = in1 ? gv : 0.0f;
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[k], b[k], acc, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) sh[w][((r / 4) * 8 + hi * 4 + (r % 4)) * C + co] = acc[r];
+    __syncthreads();
+    for (int i = threadIdx.x; i < C1_PART; i += TB)
+        part[(size_t)blockIdx.x * C1_PART + i] = ((sh[0][i] + sh[1][i]) + sh[2][i]) + sh[3][i];
 }
 
 // Sum block partials (fixed order) and scatter into the gradient vector.
-// mode 0: 32-channel layer: part [nblk][27][32 ci][32 co] (+ pb [nblk][32])
+// A thread takes four neighbouring sums of every RG-th partial, the RG
+// threads of those sums meet in LDS: the partials are read by enough threads
+// to stream them (one thread per sum over all of them took 238 us for the
+// 1024 partials of a 64^3 layer).
+// mode 0: 32-channel layer: part [nblk][27][32 ci][32 co] + bias [32]
 //         -> G[off + (t*32+ci)*32+co], G[off + 27*1024 + co] (bias)
 // mode 1: final layer (co < 2): -> G[OFF_W6 + (t*32+ci)*2+co], G[OFF_B6+co]
 // mode 2: layer 1: part [nblk][27*32 + 32] -> G[OFF_W1..], G[OFF_B1..]
-__global__ void reduce_wgrad(const float *__restrict__ part, const float *__restrict__ pb, int nblk, int mode, long off,
-                             float *__restrict__ G) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (mode == 2) {
-        if (i >= NT * C + C) return;
-        float s = 0.0f;
-        for (int b = 0; b < nblk; b++) s += part[(size_t)b * (NT * C + C) + i];
-        G[(i < NT * C ? OFF_W1 + i : OFF_B1 + (i - NT * C))] = s;
-        return;
+constexpr int RG = 16;
+__global__ void __launch_bounds__(TB)
+reduce_wgrad(const float *__restrict__ part, int nblk, int size, int mode, long off, float *__restrict__ G) {
+    __shared__ float4 sh[RG][TB / RG];
+    const int u = threadIdx.x % (TB / RG), grp = threadIdx.x / (TB / RG);
+    const int i4 = blockIdx.x * (TB / RG) + u;
+    float4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (i4 * 4 < size) {
+        const float4 *p = reinterpret_cast<const float4 *>(part) + i4;
+        const long st = size / 4;
+#pragma unroll 8
+        for (int b = grp; b < nblk; b += RG) {
+            const float4 v = p[b * st];
+            s.x += v.x;
+            s.y += v.y;
+            s.z += v.z;
+            s.w += v.w;
+        }
     }
-    long per = (long)NT * C * C;
-    if (i < per) {
-        int co = (int)(i % C);
-        if (mode == 1 && co >= 2) return;
-        float s = 0.0f;
-        for (int b = 0; b < nblk; b++) s += part[(size_t)b * per + i];
-        if (mode == 0) G[off + i] = s;
-        else G[OFF_W6 + (i / C) * 2 + co] = s;
-    } else if (i < per + C) {
-        int co = (int)(i - per);
-        if (mode == 1 && co >= 2) return;
-        float s = 0.0f;
-        for (int b = 0; b < nblk; b++) s += pb[(size_t)b * C + co];
-        if (mode == 0) G[off + per + co] = s;
-        else G[OFF_B6 + co] = s;
+    sh[grp][u] = s;
+    __syncthreads();
+    if (grp || i4 * 4 >= size) return;
+    float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < RG; k++) {
+        const float4 v = sh[k][u];
+        o[0] += v.x;
+        o[1] += v.y;
+        o[2] += v.z;
+        o[3] += v.w;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int i = i4 * 4 + e;
+        if (mode == 2) G[i < NT * C ? OFF_W1 + i : OFF_B1 + (i - NT * C)] = o[e];
+        else if (mode == 0) G[off + i] = o[e];
+        else if (i % C < 2) G[i < NT * C * C ? OFF_W6 + (i / C) * 2 + i % C : OFF_B6 + i % C] = o[e];
     }
 }
 
@@ -827,9 +970,9 @@ struct CnnWork {
     __bf16 *act[6];     // layer outputs 1..5 (act[1..5]); act[0] unused
     float *y;           // [V][2]
     __bf16 *gA, *gB;    // gradient ping-pong [V][32]
-    float *part, *pb;
+    float *part;
     double *red, *dsum;
-    long nblk_wg;
+    int nblk_wg;
 };
 
 int cnn_work(sh_ctx *ctx, long n, bool train, CnnWork &W, int n1, int n2, int n3) {
@@ -854,10 +997,9 @@ int cnn_work(sh_ctx *ctx, long n, bool train, CnnWork &W, int n1, int n2, int n3
     if (train) {
         W.gA = (__bf16 *)p; p += actsz;
         W.gB = (__bf16 *)p; p += actsz;
-        long nb = (long)ceil_div(n1, WG_X) * ceil_div(n2, WG_Y) * n3;
-        W.nblk_wg = nb;
-        SH_TRY(sh_slot(ctx, SLOT_INTERP0 + 13, (size_t)nb * (NT * C * C + C) * sizeof(float), (void **)&W.part));
-        W.pb = W.part + (size_t)nb * NT * C * C;
+        const long tiles = (long)ceil_div(n1, WG_X) * ceil_div(n2, WG_Y) * n3;
+        W.nblk_wg = (int)std::min<long>(tiles, WG_BLOCKS);
+        SH_TRY(sh_slot(ctx, SLOT_INTERP0 + 13, (size_t)W.nblk_wg * WG_PART * sizeof(float), (void **)&W.part));
         SH_TRY(sh_slot(ctx, SLOT_INTERP0 + 14, (size_t)ceil_div(n, TB) * sizeof(double) + 64, (void **)&W.red));
         W.dsum = W.red + ceil_div(n, TB);
     }
@@ -1011,19 +1153,24 @@ int sh_cnn_grad(sh_ctx *ctx, const float *params, const float *x, float xscale, 
         SH_HIP(ctx, hipStreamSynchronize(ctx->stream));
         *loss = h * (double)scale;
     }
-    unsigned gwg = (unsigned)W.nblk_wg;
-    int nred = ceil_div(per + C, TB);
+    static_assert(WG_PART % 4 == 0 && C1_PART % 4 == 0, "the partials are read as float4");
+    const int nred = ceil_div(WG_PART / 4, TB / RG);
     // layer 6 (input act5, output gradient gA)
     __bf16 *g = W.gA, *gn = W.gB;
     for (int l = 6; l >= 2; l--) {
         const __bf16 *ain = W.act[l - 1];
+        const int dl = D[l - 1];
         PROF_A(ctx);
-        hipLaunchKernelGGL(conv32_wgrad, dim3(gwg), dim3(TB), 0, ctx->stream, ain, g, W.part, W.pb, n1, n2, n3,
-                           D[l - 1]);
+        if (dl == 1)
+            hipLaunchKernelGGL(conv32_wgrad<true>, dim3(W.nblk_wg), dim3(WG_TB), 0, ctx->stream, ain, g,
+                               W.part, n1, n2, n3, dl);
+        else
+            hipLaunchKernelGGL(conv32_wgrad<false>, dim3(W.nblk_wg), dim3(WG_TB), 0, ctx->stream, ain, g,
+                               W.part, n1, n2, n3, dl);
         PROF_B(ctx, "conv32_wgrad", (double)n * 128.0);
         SH_TRY(sh_launch_check(ctx, "conv32_wgrad"));
-        hipLaunchKernelGGL(reduce_wgrad, dim3(nred), dim3(TB), 0, ctx->stream, W.part, W.pb, (int)gwg, l == 6 ? 1 : 0,
-                           l == 6 ? 0L : OFF_L(l), grad);
+        hipLaunchKernelGGL(reduce_wgrad, dim3(nred), dim3(TB), 0, ctx->stream, W.part, W.nblk_wg, WG_PART,
+                           l == 6 ? 1 : 0, l == 6 ? 0L : OFF_L(l), grad);
         SH_TRY(sh_launch_check(ctx, "reduce_wgrad"));
         // input gradient through the ReLU of layer l-1
         SH_TRY(conv_launch(ctx, 2, g, W.Wb + (size_t)(l - 2) * per, nullptr, gn, ain, n1, n2, n3, D[l - 1],
@@ -1031,14 +1178,12 @@ int sh_cnn_grad(sh_ctx *ctx, const float *params, const float *x, float xscale, 
         std::swap(g, gn);
     }
     // layer 1 weights
-    int vpb = 256;
-    int nb1 = ceil_div(n, vpb);
-    SH_TRY(sh_slot(ctx, SLOT_INTERP0 + 15, (size_t)nb1 * (NT * C + C) * sizeof(float), (void **)&W.part));
-    hipLaunchKernelGGL(conv1_wgrad, dim3(nb1), dim3(1024), 0, ctx->stream, x, xscale, g, W.part, n1, n2, n3, vpb,
-                       D[0]);
+    const int nb1 = (int)std::min<long>(ceil_div((long)n2 * n3, 4), C1_BLOCKS);
+    SH_TRY(sh_slot(ctx, SLOT_INTERP0 + 15, (size_t)nb1 * C1_PART * sizeof(float), (void **)&W.part));
+    hipLaunchKernelGGL(conv1_wgrad, dim3(nb1), dim3(TB), 0, ctx->stream, x, xscale, g, W.part, n1, n2, n3, D[0]);
     SH_TRY(sh_launch_check(ctx, "conv1_wgrad"));
-    hipLaunchKernelGGL(reduce_wgrad, dim3(ceil_div(NT * C + C, TB)), dim3(TB), 0, ctx->stream, W.part, nullptr, nb1, 2,
-                       0L, grad);
+    hipLaunchKernelGGL(reduce_wgrad, dim3(ceil_div(C1_PART / 4, TB / RG)), dim3(TB), 0, ctx->stream, W.part, nb1,
+                       C1_PART, 2, 0L, grad);
     return sh_launch_check(ctx, "reduce_wgrad");
 }
 

@@ -94,6 +94,21 @@ def test_gradient_matches_oracle(ws, shape):
     assert abs(loss2 - l2) <= 1e-3 * abs(l2)
 
 
+# edges of the weight-gradient tiles (64 x 4 voxels): one voxel short of and
+# past a tile, fewer voxels than a fragment, and more tiles than blocks; the
+# bar leaves room for gradients that round to the other bfloat16 neighbour
+# (2^-8 relative for single voxels), a lost or doubled voxel row exceeds it
+@pytest.mark.parametrize("shape,dil", [((64, 4, 3), None), ((63, 5, 2), None), ((65, 3, 70), None), ((2, 1, 1), None),
+                                       ((17, 9, 1), (2, 1, 3, 8, 1, 2))])
+def test_weight_gradient_tile_edges(ws, shape, dil):
+    p, x, t, wt = _case(6, shape)
+    _, g = ws.cnn_grad(_dev(p), _dev(x), shape, 0.5, _dev(t), _dev(wt), dil=dil)
+    _, gref = K.loss_and_grad(p, x, t, shape, wt=wt, xscale=0.5, quant=True, dil=dil)
+    g = g.cpu().numpy()
+    for name, sl in _blocks().items():
+        assert _rel(g[sl], gref[sl]) <= 1e-2, name
+
+
 @pytest.mark.parametrize("dil", [(1, 2, 4, 8, 2, 1), (3, 1, 2, 1, 5, 2)])
 def test_dilated_forward_and_gradient(ws, dil):
     shape = (70, 21, 18)
