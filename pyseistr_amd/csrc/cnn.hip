@@ -1016,7 +1016,12 @@ int conv_launch(sh_ctx *ctx, int mode, const __bf16 *in, const __bf16 *Wg, const
     // (the plane-scatter kernel addresses its buffers with 32-bit offsets)
     if (dil == 1 && kind == 'z' && (double)n1 * n2 * n3 * 64.0 < 4.0e9) {
         long ntiles = (long)ceil_div(n1, 64) * ceil_div(n2, CW) * n3;
-        dim3 grid((unsigned)std::min<long>(ntiles, 1024));
+        // one block of 8 waves fits a CU: with fewer tiles than 4 per CU a
+        // block takes at least two planes, so that it stages its weights
+        // and reads shared input planes once for both (64^3: 512 tiles over
+        // 256 blocks 28 us, over 512 blocks 40 us; over 128 blocks 36 us)
+        const long want = std::max<long>(256, std::min<long>(1024, ntiles / 2));
+        dim3 grid((unsigned)std::min<long>(ntiles, want));
         PROF_A(ctx);
         if (mode == 0)
             hipLaunchKernelGGL((conv32z<0>), grid, dim3(CTB), 0, ctx->stream, in, Wg, bias, out, aux, n1, n2, n3);
