@@ -7,6 +7,7 @@ HIPCC=${HIPCC:-/opt/rocm/bin/hipcc}
 JOBS=${JOBS:-8}
 SRCS="common dip"
 [ -f "$HERE/spray.hip" ] && SRCS="$SRCS spray"
+[ -f "$HERE/chain2.hip" ] && SRCS="$SRCS chain2"
 [ -f "$HERE/interp.hip" ] && SRCS="$SRCS interp"
 [ -f "$HERE/cnn.hip" ] && SRCS="$SRCS cnn"
 [ -f "$HERE/batch.hip" ] && SRCS="$SRCS batch"

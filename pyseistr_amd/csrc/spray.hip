@@ -608,15 +608,17 @@ spray2_adj(const float *__restrict__ U, const float *__restrict__ dip, const flo
 
 // x = ((x or 0) + chain_right) + chain_left + centre: the accumulation
 // order of the adjoint spray (sof_cfuns.c:969-995).  C[0] holds the chains
-// from the left (dir 0), C[1] those from the right (dir 1).
-__global__ void spray2_adj_combine(const float *__restrict__ C, const float *__restrict__ U, float *__restrict__ x,
+// from the left (dir 0), C[1] those from the right (dir 1).  The centre is
+// U's centre slot, or with ww that of the weighted field U (chain2_adj).
+__global__ void spray2_adj_combine(const float *__restrict__ C, const float *U, const float *__restrict__ ww, float *x,
                                    long n, int ns, int add) {
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    const float c = ww ? U[i] * (float)(ns + 1) * ww[i] : U[(long)ns * n + i];
     float v = add ? x[i] : 0.0f;
     v = v + C[n + i];
     v = v + C[i];
-    v = v + U[(long)ns * n + i];
+    v = v + c;
     x[i] = v;
 }
 
@@ -950,6 +952,33 @@ bool spray2_buf(int n1, long n, int ns, int order, long nthr) {
         }                                    \
     } while (0)
 
+// The chains run by blocks of threads (chain2.hip) where a trace fits
+// their LDS, by one thread each otherwise; the switches of the
+// one-thread-per-chain kernels select those.
+bool spray2_blocks(const Pwsmooth2 &P) {
+    return !getenv("SH_SPRAY2_PF") && !getenv("SH_SPRAY2_BUF") && !getenv("SH_SPRAY2_TB") &&
+           chain2_fits(P.n1, P.n2, P.n3, P.order);
+}
+
+// Adjoint chains of P from the slots U, or from the field U weighted by ww
+// (only where the block kernels run), into P.C.
+int pws2_adjoint(sh_ctx *ctx, Pwsmooth2 &P, bool blocks, const float *U, const float *ww) {
+    const long n = (long)P.n1 * P.n2 * P.n3;
+    PROF_A(ctx);
+    if (blocks) {
+        SH_TRY(chain2_adjoint(ctx, P, U, ww));
+    } else {
+        const int TB2 = spray2_tb();
+        dim3 grid(ceil_div(2L * P.n2, TB2), P.n3);
+        const bool buf = spray2_buf(P.n1, n, P.ns, P.order, P.nthr);
+        SPRAY2_BUF_DISPATCH(BUF, buf, SPRAY2_PF_DISPATCH(PF, false, SH_DISPATCH_NW(ctx, P.order, NW,
+                       hipLaunchKernelGGL((spray2_adj<BUF, NW, PF>), grid, dim3(TB2), 0, ctx->stream, U, P.dip, P.F,
+                                          P.C, P.n1, P.n2, P.n3, P.ns, P.e, P.scr, P.tr, P.nthr, P.stop))));
+    }
+    PROF_B(ctx, "spray2_adj", 12.0 * 2 * P.ns * (double)n);
+    return sh_launch_check(ctx, "spray2_adj");
+}
+
 // Factor cache of P into caller-provided buffers: scr holds 2*nthr*n1
 // floats (solver scratch, then the running trace planes), F
 // 3 * fac_plane_floats(2 * order, n): the two factor variants, then the
@@ -987,13 +1016,17 @@ int pws2_prepare(sh_ctx *ctx, Pwsmooth2 &P, int slot_scr, int slot_F) {
 // launch (it uses the scratch plane P.tr, free outside the adjoint), so
 // two latency-bound sets of chains run side by side.
 int pws2_spray(sh_ctx *ctx, Pwsmooth2 &P, const float *x, const float *x2 = nullptr, float *U2 = nullptr) {
-    const int TB2 = spray2_tb();
-    dim3 grid(ceil_div(2L * P.n2, TB2), P.n3, x2 ? 2 : 1);
     PROF_A(ctx);
-    const bool buf = spray2_buf(P.n1, (long)P.n1 * P.n2 * P.n3, P.ns, P.order, P.nthr);
-    SPRAY2_BUF_DISPATCH(BUF, buf, SPRAY2_PF_DISPATCH(PF, true, SH_DISPATCH_NW(ctx, P.order, NW,
-                   hipLaunchKernelGGL((spray2_fwd<BUF, NW, PF>), grid, dim3(TB2), 0, ctx->stream, x, P.dip, P.F, P.U,
-                                      P.n1, P.n2, P.n3, P.ns, P.e, P.scr, P.nthr, P.stop, x2, U2))));
+    if (spray2_blocks(P)) {
+        SH_TRY(chain2_forward(ctx, P, x, x2, U2));
+    } else {
+        const int TB2 = spray2_tb();
+        dim3 grid(ceil_div(2L * P.n2, TB2), P.n3, x2 ? 2 : 1);
+        const bool buf = spray2_buf(P.n1, (long)P.n1 * P.n2 * P.n3, P.ns, P.order, P.nthr);
+        SPRAY2_BUF_DISPATCH(BUF, buf, SPRAY2_PF_DISPATCH(PF, true, SH_DISPATCH_NW(ctx, P.order, NW,
+                       hipLaunchKernelGGL((spray2_fwd<BUF, NW, PF>), grid, dim3(TB2), 0, ctx->stream, x, P.dip, P.F,
+                                          P.U, P.n1, P.n2, P.n3, P.ns, P.e, P.scr, P.nthr, P.stop, x2, U2))));
+    }
     PROF_B(ctx, "spray2_fwd", (x2 ? 2 : 1) * 12.0 * 2 * P.ns * (double)P.n1 * P.n2 * P.n3);
     return sh_launch_check(ctx, "spray2_fwd");
 }
@@ -1055,25 +1088,18 @@ int pws2_apply(sh_ctx *ctx, Pwsmooth2 &P, int adj, int add, float *trace, float 
         PROF_B(ctx, "pwsmooth_fwd", 4.0 * (ns2 + 2 + add) * (double)n);
         return sh_launch_check(ctx, "pwsmooth_fwd");
     }
-    {
+    const bool blocks = spray2_blocks(P);
+    if (!blocks) {
         PROF_A(ctx);
         hipLaunchKernelGGL(pwsmooth_adj_weight, dim3(g), dim3(TB), 0, ctx->stream, smooth, P.ww, P.U, n, P.ns);
         PROF_B(ctx, "pwsmooth_adj_weight", 4.0 * (ns2 + 2) * (double)n);
+        SH_TRY(sh_launch_check(ctx, "pwsmooth_adj_weight"));
     }
-    SH_TRY(sh_launch_check(ctx, "pwsmooth_adj_weight"));
-    const int TB2 = spray2_tb();
-    dim3 grid(ceil_div(2L * P.n2, TB2), P.n3);
-    {
-        PROF_A(ctx);
-        const bool buf = spray2_buf(P.n1, n, P.ns, P.order, P.nthr);
-        SPRAY2_BUF_DISPATCH(BUF, buf, SPRAY2_PF_DISPATCH(PF, false, SH_DISPATCH_NW(ctx, P.order, NW,
-                       hipLaunchKernelGGL((spray2_adj<BUF, NW, PF>), grid, dim3(TB2), 0, ctx->stream, P.U, P.dip, P.F,
-                                          P.C, P.n1, P.n2, P.n3, P.ns, P.e, P.scr, P.tr, P.nthr, P.stop))));
-        PROF_B(ctx, "spray2_adj", 12.0 * 2 * P.ns * (double)n);
-    }
-    SH_TRY(sh_launch_check(ctx, "spray2_adj"));
+    // the block kernels weight the field where they read it
+    const float *src = blocks ? smooth : P.U, *ww = blocks ? P.ww : nullptr;
+    SH_TRY(pws2_adjoint(ctx, P, blocks, src, ww));
     PROF_A(ctx);
-    hipLaunchKernelGGL(spray2_adj_combine, dim3(g), dim3(TB), 0, ctx->stream, P.C, P.U, trace, n, P.ns, add);
+    hipLaunchKernelGGL(spray2_adj_combine, dim3(g), dim3(TB), 0, ctx->stream, P.C, src, ww, trace, n, P.ns, add);
     PROF_B(ctx, "spray2_adj_combine", 4.0 * (4 + add) * (double)n);
     return sh_launch_check(ctx, "spray2_adj_combine");
 }
@@ -1356,14 +1382,9 @@ int shd_pwspray2d(sh_ctx *ctx, int adj, const float *dip, int n1, int n2, int ns
                                      (size_t)n1 * sizeof(float), (size_t)n2, hipMemcpyDeviceToDevice, ctx->stream));
         SH_TRY(transpose(ctx, tmp, P.U + (long)s * n, n1, n2, true));
     }
-    const int TB2 = spray2_tb();
-    dim3 grid(ceil_div(2L * n2, TB2), 1);
-    const bool buf = spray2_buf(n1, n, ns, order, P.nthr);
-    SPRAY2_BUF_DISPATCH(BUF, buf, SPRAY2_PF_DISPATCH(PF, false, SH_DISPATCH_NW(ctx, order, NW,
-                   hipLaunchKernelGGL((spray2_adj<BUF, NW, PF>), grid, dim3(TB2), 0, ctx->stream, P.U, P.dip, P.F, P.C,
-                                      n1, n2, 1, ns, P.e, P.scr, P.tr, P.nthr, nullptr))));
-    SH_TRY(sh_launch_check(ctx, "spray2_adj"));
-    hipLaunchKernelGGL(spray2_adj_combine, dim3(ceil_div(n, TB)), dim3(TB), 0, ctx->stream, P.C, P.U, xT, n, ns, 0);
+    SH_TRY(pws2_adjoint(ctx, P, spray2_blocks(P), P.U, nullptr));
+    hipLaunchKernelGGL(spray2_adj_combine, dim3(ceil_div(n, TB)), dim3(TB), 0, ctx->stream, P.C, P.U, nullptr, xT, n,
+                       ns, 0);
     SH_TRY(sh_launch_check(ctx, "spray2_adj_combine"));
     return transpose(ctx, xT, x, n1, n2, false);
 }

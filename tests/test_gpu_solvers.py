@@ -134,6 +134,31 @@ def test_spray2_prefetch_distances_identical(ps, monkeypatch):
         same(a, c, f"call {k}, pointers")
 
 
+@pytest.mark.parametrize("n1,n2,n3,ns,order", [(8, 1, 1, 2, 1), (9, 2, 3, 3, 2), (17, 5, 1, 6, 4), (31, 33, 2, 2, 3),
+                                                (300, 17, 1, 4, 2), (515, 40, 1, 3, 2), (1030, 9, 1, 2, 3),
+                                                (2100, 6, 1, 2, 2), (4000, 5, 1, 1, 1), (33, 70, 33, 2, 2)])
+def test_chain_blocks_equal_single_threads(ps, monkeypatch, n1, n2, n3, ns, order):
+    """The spray chains by blocks of threads and one thread each
+    (SH_SPRAY2_PF selects the latter) give the same bits: one trace, fewer
+    traces than radii, pieces and blocks that do not divide, traces too long
+    for the blocks, and enough chains for the long pieces."""
+    from pyseistr_amd import filters
+    rng = np.random.default_rng(n1 + n2)
+    d = rng.standard_normal((n1, n2, n3)).astype(np.float32)
+    p = rng.uniform(-2, 2, (n1, n2, n3)).astype(np.float32)
+    u = rng.standard_normal(n1 * n2 * (2 * ns + 1)).astype(np.float32)
+
+    def calls():
+        return [filters.pwspray2d(d[:, :, 0], p[:, :, 0], ns, order, 0.01),
+                filters.pwspray2d_adjoint(u, p[:, :, 0], ns, order, 0.01, (n1, n2)),
+                ps.somean2dc(d, p, ns, order, 0.01), ps.somean2dc(d, p, ns, order, 0.01, adj=1)]
+
+    a = calls()
+    monkeypatch.setenv("SH_SPRAY2_PF", "8")
+    for k, (x, y) in enumerate(zip(a, calls())):
+        same(x, y, f"call {k}")
+
+
 def test_spray3_level_paths_identical(ps, monkeypatch):
     """The 3-D spray levels give the same bits through buffer resources (the
     default) and through pointers (SH_SPRAY_BUF=0), at every prefetch
