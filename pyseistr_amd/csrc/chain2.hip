@@ -425,11 +425,124 @@ chain2_adj(const float *__restrict__ U, const float *__restrict__ ww, const floa
     }
 }
 
+// The chains' factors (factor_sweep's, identical), in two launches: the
+// normal matrix's rows by one thread per 16 samples of a trace and direction,
+// written where the factor will be, then the LDL^T recurrence alone, one
+// thread per trace, in place with the rows loaded 8 samples ahead.  As one
+// sweep per trace, forming the rows was half of its instructions.
+constexpr int FR = 16;
+template <int NW>
+__global__ void __launch_bounds__(256)
+chain2_rows(const float *__restrict__ dip, float *__restrict__ F, int n1, int n2, int n3, float e, int np) {
+    constexpr int NA = 2 * NW + 1, NB = 2 * NW;
+    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)(gid % n2), vc = (int)(gid / n2), v = vc / np, k0 = vc % np * FR;
+    if (v > 1 || (v == 0 ? i > n2 - 2 : i < 1)) return;  // never a target in that direction
+    const long slice = (long)n1 * n2, base = blockIdx.y * slice, n = slice * n3;
+    const Acc q{dip + base + (v == 0 ? i : i - 1), n2};
+    const FactorOut Fs = fac_out_at(F + v * fac_plane_floats(NB, n), NB, n, base + i, n2);
+    float A[NA][NA];
+#pragma unroll
+    for (int w = 0; w < NA; w++) taps_at<NW>(q, k0 - NW + w, n1, v == 1, A[w]);
+    for (int k = k0; k < min(k0 + FR, n1); k++) {
+        float diag, offd[NB];
+        reg_row<NB>(k, n1, e, diag, offd);
+#pragma unroll
+        for (int j = 0; j < NA; j++) {
+            const int kk = k + j - NW;
+            if (kk >= NW && kk < n1 - NW) diag += A[j][j] * A[j][j];
+        }
+#pragma unroll
+        for (int m = 0; m < NB; m++)
+#pragma unroll
+            for (int j = m + 1; j < NA; j++) {
+                const int kk = k + j - NW;
+                if (kk >= NW && kk < n1 - NW) offd[m] += A[j][j - m - 1] * A[j][j];
+            }
+        fac_put<NB>(Fs, k, diag, offd);
+#pragma unroll
+        for (int w = 0; w < NA - 1; w++)
+#pragma unroll
+            for (int j = 0; j < NA; j++) A[w][j] = A[w + 1][j];
+        taps_at<NW>(q, k + 1 + NW, n1, v == 1, A[NA - 1]);
+    }
+}
+
+template <int NW>
+__global__ void __launch_bounds__(64)
+chain2_ldl(float *__restrict__ F, int n1, int n2, int n3) {
+    constexpr int NB = 2 * NW, D = 8;
+    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)(gid % n2), v = (int)(gid / n2);
+    if (v > 1 || (v == 0 ? i > n2 - 2 : i < 1)) return;
+    const long slice = (long)n1 * n2, base = blockIdx.y * slice, n = slice * n3;
+    float *const Fv = F + v * fac_plane_floats(NB, n);
+    const FactorOut Fo = fac_out_at(Fv, NB, n, base + i, n2);
+    const Factor Fi{Fo.d, Fo.o, n2};
+    float rd[D], ro[D][NB], Ld[NB], Lo[NB][NB];
+    auto fetch = [&](int s, int k) {
+        const long kc = k < n1 ? k : n1 - 1;
+        rd[s] = fac_d(Fi, kc);
+        fac_row<NB>(Fi, kc, ro[s]);
+    };
+#pragma unroll
+    for (int r = 0; r < NB; r++) {
+        Ld[r] = 0.0f;
+#pragma unroll
+        for (int m = 0; m < NB; m++) Lo[r][m] = 0.0f;
+    }
+#pragma unroll
+    for (int s = 0; s < D; s++) fetch(s, s);
+    auto step = [&](int s, int k) {
+        // rows before the trace are zeros: subtracting 0 * 0 * 0 changes nothing
+        float t = rd[s];
+#pragma unroll
+        for (int m = 0; m < NB; m++) t -= (Lo[m][m]) * (Lo[m][m]) * (Ld[m]);
+        float ok[NB];
+#pragma unroll
+        for (int c = 0; c < NB; c++) {
+            float w = ro[s][c];
+#pragma unroll
+            for (int m = 0; m < NB - c - 1; m++) w -= (Lo[m][m]) * (Lo[m][c + m + 1]) * (Ld[m]);
+            ok[c] = c < n1 - k - 1 ? w / t : 0.0f;
+        }
+        fac_put<NB>(Fo, k, t, ok);
+#pragma unroll
+        for (int r = NB - 1; r > 0; r--) {
+            Ld[r] = Ld[r - 1];
+#pragma unroll
+            for (int m = 0; m < NB; m++) Lo[r][m] = Lo[r - 1][m];
+        }
+        Ld[0] = t;
+#pragma unroll
+        for (int m = 0; m < NB; m++) Lo[0][m] = ok[m];
+        fetch(s, k + D);
+    };
+    int k0 = 0;
+    for (; k0 + D <= n1; k0 += D) {
+#pragma unroll
+        for (int s = 0; s < D; s++) step(s, k0 + s);
+    }
+#pragma unroll
+    for (int s = 0; s < D; s++)
+        if (k0 + s < n1) step(s, k0 + s);
+}
+
 }  // namespace
 
 bool chain2_fits(int n1, int n2, int n3, int order) {
     // (a slice's factor rows are addressed with 32-bit offsets)
     return n3 <= 65535 && (double)n1 * n2 * 8 * order < 4294967295.0 && chain_plan(n1, n2, n3, order).nt > 0;
+}
+
+int chain2_factor(sh_ctx *ctx, const Pwsmooth2 &P) {
+    const int np = ceil_div(P.n1, FR);
+    SH_DISPATCH_NW(ctx, P.order, NW,
+                   hipLaunchKernelGGL((chain2_rows<NW>), dim3(ceil_div(2L * P.n2 * np, 256), P.n3), dim3(256), 0,
+                                      ctx->stream, P.dip, P.F, P.n1, P.n2, P.n3, P.e, np);
+                   hipLaunchKernelGGL((chain2_ldl<NW>), dim3(ceil_div(2L * P.n2, 64), P.n3), dim3(64), 0, ctx->stream,
+                                      P.F, P.n1, P.n2, P.n3));
+    return sh_launch_check(ctx, "chain2_factor");
 }
 
 // NW and D of a plan (orders 3 and 4 keep a ring of 8 rows)

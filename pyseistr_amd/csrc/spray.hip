@@ -960,35 +960,17 @@ bool spray2_blocks(const Pwsmooth2 &P) {
            chain2_fits(P.n1, P.n2, P.n3, P.order);
 }
 
-// Adjoint chains of P from the slots U, or from the field U weighted by ww
-// (only where the block kernels run), into P.C.
-int pws2_adjoint(sh_ctx *ctx, Pwsmooth2 &P, bool blocks, const float *U, const float *ww) {
-    const long n = (long)P.n1 * P.n2 * P.n3;
-    PROF_A(ctx);
-    if (blocks) {
-        SH_TRY(chain2_adjoint(ctx, P, U, ww));
-    } else {
-        const int TB2 = spray2_tb();
-        dim3 grid(ceil_div(2L * P.n2, TB2), P.n3);
-        const bool buf = spray2_buf(P.n1, n, P.ns, P.order, P.nthr);
-        SPRAY2_BUF_DISPATCH(BUF, buf, SPRAY2_PF_DISPATCH(PF, false, SH_DISPATCH_NW(ctx, P.order, NW,
-                       hipLaunchKernelGGL((spray2_adj<BUF, NW, PF>), grid, dim3(TB2), 0, ctx->stream, U, P.dip, P.F,
-                                          P.C, P.n1, P.n2, P.n3, P.ns, P.e, P.scr, P.tr, P.nthr, P.stop))));
-    }
-    PROF_B(ctx, "spray2_adj", 12.0 * 2 * P.ns * (double)n);
-    return sh_launch_check(ctx, "spray2_adj");
-}
-
 // Factor cache of P into caller-provided buffers: scr holds 2*nthr*n1
 // floats (solver scratch, then the running trace planes), F
 // 3 * fac_plane_floats(2 * order, n): the two factor variants, then the
-// filter taps of the slopes.
+// filter taps of the slopes (which the block kernels form themselves).
 int pws2_prepare_bufs(sh_ctx *ctx, Pwsmooth2 &P, float *scr, float *F) {
     long n = (long)P.n1 * P.n2 * P.n3;
     P.nthr = pws2_nthr(P.n2, P.n3);
     P.scr = scr;
     P.tr = P.scr + (long)P.nthr * P.n1;
     P.F = F;
+    if (spray2_blocks(P)) return chain2_factor(ctx, P);
     const int TB2 = spray2_tb();
     dim3 grid(ceil_div(2L * P.n2, TB2), P.n3);
     PROF_A(ctx);
@@ -1010,6 +992,25 @@ int pws2_prepare(sh_ctx *ctx, Pwsmooth2 &P, int slot_scr, int slot_F) {
     SH_TRY(sh_slot(ctx, slot_scr, (size_t)nthr * P.n1 * 2 * sizeof(float), (void **)&scr));
     SH_TRY(sh_slot(ctx, slot_F, (size_t)3 * fac_plane_floats(2 * P.order, n) * sizeof(float), (void **)&F));
     return pws2_prepare_bufs(ctx, P, scr, F);
+}
+
+// Adjoint chains of P from the slots U, or from the field U weighted by ww
+// (only where the block kernels run), into P.C.
+int pws2_adjoint(sh_ctx *ctx, Pwsmooth2 &P, bool blocks, const float *U, const float *ww) {
+    const long n = (long)P.n1 * P.n2 * P.n3;
+    PROF_A(ctx);
+    if (blocks) {
+        SH_TRY(chain2_adjoint(ctx, P, U, ww));
+    } else {
+        const int TB2 = spray2_tb();
+        dim3 grid(ceil_div(2L * P.n2, TB2), P.n3);
+        const bool buf = spray2_buf(P.n1, n, P.ns, P.order, P.nthr);
+        SPRAY2_BUF_DISPATCH(BUF, buf, SPRAY2_PF_DISPATCH(PF, false, SH_DISPATCH_NW(ctx, P.order, NW,
+                       hipLaunchKernelGGL((spray2_adj<BUF, NW, PF>), grid, dim3(TB2), 0, ctx->stream, U, P.dip, P.F,
+                                          P.C, P.n1, P.n2, P.n3, P.ns, P.e, P.scr, P.tr, P.nthr, P.stop))));
+    }
+    PROF_B(ctx, "spray2_adj", 12.0 * 2 * P.ns * (double)n);
+    return sh_launch_check(ctx, "spray2_adj");
 }
 
 // Spray of x into P.U; with x2 also the spray of x2 into U2 in the same
