@@ -11,7 +11,7 @@
 //  * the triangle smoother is the direct (2nb-1)-tap stencil with even
 //    reflection, staged through LDS tiles with halos, the vector updates of
 //    the CG fused into the first/last smoothing pass.
-#include "dipcore.hpp"
+#include "dip2.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -1043,6 +1043,35 @@ extern "C" int shd_dip(sh_ctx *ctx, const float *data, const float *mask, const 
         // no better), so it stays opt-in.
         if (env && env[0] == '3' && plan.naxes == 3 && plan.r[1] - 1 <= P_HMAX2 && plan.r[2] >= 2 && plan.r[2] <= 7)
             plan.fused = 3;
+    }
+    // a 2-D section that fits the chip: resident, in one launch (dip2.hip).
+    // The switches of the smoothing passes select the launches.
+    if (n3 == 1 && r3 <= 1 && !getenv("SH_SMOOTH_FUSED") && !getenv("SH_SMOOTH_TILE") && !getenv("SH_SMOOTH_WAVE") &&
+        !getenv("SH_SMOOTH_COL")) {
+        unsigned char *m0 = nullptr;
+        if (mask) {
+            SH_TRY(sh_slot(ctx, SLOT_DIP0 + 1, (size_t)g.n * 2, (void **)&m0));
+            hipLaunchKernelGGL(mask_kernel, dim3(ceil_div(g.n, 256)), dim3(256), 0, ctx->stream, mask, m0, m0 + g.n, n1,
+                               n2, n3, order);
+            SH_TRY(sh_launch_check(ctx, "mask_kernel"));
+        }
+        int *rec = nullptr, ran = 0;
+        if (rep) SH_TRY(sh_slot(ctx, SLOT_DIP0 + 4, REC_INTS * sizeof(int), (void **)&rec));
+        SH_TRY(dip2_resident(ctx, n1, n2, plan.r[0], plan.r[1], order, data, m0, init, niter, liter, rec, dip, &ran));
+        if (ran) {
+            if (rep) {
+                int h[REC_INTS];
+                rep->ndir = 1;
+                rep->niter = niter;
+                SH_HIP(ctx, hipMemcpyAsync(h, rec, sizeof h, hipMemcpyDeviceToHost, ctx->stream));
+                SH_HIP(ctx, hipStreamSynchronize(ctx->stream));
+                for (int it = 0; it < niter && it < 64; it++) {
+                    rep->cg_iters[0][it] = h[2 * it];
+                    rep->ls_step[0][it] = h[2 * it + 1];
+                }
+            }
+            return SH_OK;
+        }
     }
     if (plan.naxes == 0) {  // no smoothing: identity through a 1-tap pass
         plan.naxes = 1;

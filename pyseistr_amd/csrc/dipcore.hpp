@@ -31,7 +31,7 @@ struct DipScal {
     int rec[2 * 64];    // per GN iteration (first 64): cg iterations, accepted step
 };
 
-enum { F_USUM = 0, F_DIVN, F_R0, F_GN, F_BETA, F_LS };
+enum { F_USUM = 0, F_DIVN, F_R0, F_GN, F_BETA, F_LS, F_LS0, F_LS7 };
 
 // fold position q (may lie outside [0,n)) back by even reflection
 __device__ inline int fold_idx(int q, int n) {
@@ -102,6 +102,33 @@ __device__ inline void dip_scalar_step(DipScal *sc, const double *tot, int mode,
             if (it < 64) {
                 sc->rec[2 * it] = sc->cg_iters;
                 sc->rec[2 * it + 1] = sc->ls_k;
+            }
+        }
+        break;
+    case F_LS0:  // the full step alone
+        if (tot[0] < sc->usum) {
+            sc->accepted = 1;
+            sc->ls_k = 0;
+            sc->usum = tot[0];
+            if (it < 64) {
+                sc->rec[2 * it] = sc->cg_iters;
+                sc->rec[2 * it + 1] = 0;
+            }
+        }
+        break;
+    case F_LS7:  // the seven halved steps, where the full one was refused
+        if (sc->accepted) break;
+        for (int k = 1; k <= 7; k++) {
+            const bool ok = tot[k - 1] < sc->usum;
+            if (ok || k == 7) {
+                sc->accepted = ok ? 1 : 2;
+                sc->ls_k = ok ? k : 8;
+                sc->usum = tot[k - 1];
+                if (it < 64) {
+                    sc->rec[2 * it] = sc->cg_iters;
+                    sc->rec[2 * it + 1] = sc->ls_k;
+                }
+                break;
             }
         }
         break;

@@ -203,3 +203,55 @@ def test_pwd_virtual_blocks_identical(ps, monkeypatch):
         for k, ((a, ia), (b, ib)) in enumerate(zip(out["1"], out[v])):
             same(a, b, f"V={v} call {k}")
             assert ia == ib
+
+
+@pytest.mark.parametrize("shape,rect,order,masked", [((8, 2), (3, 2), 1, False), ((31, 15), (1, 1), 2, False),
+                                                     ((33, 17), (10, 20), 2, True), ((64, 32), (5, 1), 3, False),
+                                                     ((130, 70), (1, 9), 2, True), ((515, 257), (10, 20), 2, False),
+                                                     ((1030, 260), (20, 20), 1, False), ((1500, 600), (4, 4), 2, False)])
+def test_resident_section_equals_launches(ps, monkeypatch, shape, rect, order, masked):
+    """The dip of a 2-D section in one resident launch and as a sequence of
+    launches (SH_SMOOTH_WAVE selects it): the float operations are the same,
+    only double sums are added in another order, so the decisions agree and
+    the dips differ by no more than a rounding of a step length moves them.
+    Tile edges, radii past the section, one tile, every tile shape, and a
+    section with too many tiles, which takes the launches either way."""
+    rng = np.random.default_rng(shape[0])
+    d = rng.standard_normal(shape).astype(np.float32)
+    init = rng.uniform(-0.5, 0.5, shape).astype(np.float32)
+    mask = (rng.random(shape) > 0.02).astype(np.float32) if masked else None
+    kw = dict(niter=3, liter=12, order=order, rect=[rect[0], rect[1], 1], mask=mask, init=init, report=True)
+    a, ra = ps.dip2dc(d, **kw)
+    monkeypatch.setenv("SH_SMOOTH_WAVE", "1")
+    b, rb = ps.dip2dc(d, **kw)
+    assert ra["cg_iters"] == rb["cg_iters"] and ra["ls_step"] == rb["ls_step"]
+    assert np.abs(a - b).max() <= 1e-6 * max(1.0, np.abs(b).max())
+
+
+def test_resident_sections_from_threads(ps):
+    """Sections estimated at once from several threads and streams, and into
+    the data's own buffer, equal the ones estimated alone."""
+    import threading
+
+    import torch
+    from pyseistr_amd import dip
+    rng = np.random.default_rng(5)
+    shapes = [(512, 512, 1), (300, 90, 1), (512, 512, 1), (128, 64, 1)]
+    data = [torch.from_numpy(rng.standard_normal(a * b).astype(np.float32)).cuda() for a, b, _ in shapes]
+    alone = [dip.dip_device(x, s, niter=2, rect=(6, 6, 1)).cpu().numpy() for x, s in zip(data, shapes)]
+    got = [None] * len(shapes)
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(3):
+                got[k] = dip.dip_device(data[k], shapes[k], niter=2, rect=(6, 6, 1)).cpu().numpy()
+
+    torch.cuda.synchronize()
+    th = [threading.Thread(target=work, args=(k,)) for k in range(len(shapes))]
+    [t.start() for t in th]
+    [t.join() for t in th]
+    for k, (x, y) in enumerate(zip(got, alone)):
+        assert np.array_equal(x, y), k
+    buf = data[1].clone()
+    dip.dip_device(buf, shapes[1], niter=2, rect=(6, 6, 1), out=buf)
+    assert np.array_equal(buf.cpu().numpy(), alone[1])
