@@ -249,6 +249,106 @@ pwd_adj(const float *__restrict__ rr, const unsigned char *__restrict__ known,
     }
 }
 
+// The operators without drift.  Each block runs a contiguous range of
+// samples and sums once at its end: with a sum per 256 samples the wave sums
+// of the six dots were most of pwd_fwd's instructions, and adding up 23
+// thousand partials six times most of the scalar step.  The samples' float
+// operations are those of the kernels above.  301 x 101 x 97, order 2, one
+// iteration: forward 55 -> 38 us, scalars 26 -> 8 us.  What is left of the
+// forward is its five taps in double (about 100 operations a sample) and 106
+// MB of traffic (22 us); two samples a thread in flight measured 38 as well.
+template <int NW>
+__global__ void __launch_bounds__(TB)
+pwd_fwd_range(const float *__restrict__ x, float *__restrict__ y, const float *__restrict__ ss,
+              const float *__restrict__ rr, Geo g, double *part, const float *base, const SolverState *st) {
+    __shared__ double sh[16 * 6];
+    if (st && solver_done(st)) return;
+    const long ny = g.n * g.nparts, per = (ny + gridDim.x - 1) / gridDim.x;
+    const long i0 = (long)blockIdx.x * per, i1 = min(ny, i0 + per);
+    double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    for (long c = i0; c < i1; c += TB) {
+        const long i = c + threadIdx.x;
+        float v;
+        double d[6];
+        pwd_fwd_sample<NW, false>(x, ss, rr, g, base, i < i1 ? i : ny, ny, v, d);
+        if (i < i1) y[i] = v;
+#pragma unroll
+        for (int k = 0; k < 6; k++) acc[k] += d[k];
+    }
+    block_sum_multi<6>(acc, sh);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < 6; k++) part[(long)k * gridDim.x + blockIdx.x] = acc[k];
+}
+
+// The adjoint: an output gathers 2NW+1 products from each of four source
+// rows (its own trace and the one before, in both parts), and its neighbours
+// gather the same ones.  So a block forms the products of each source sample
+// once (five taps share their factors' conversions; one tap at a time they
+// were 20 a sample) for TB consecutive samples of the flat index, hands them
+// over through LDS, and the TB - 2 h inner threads (h: the reach of the
+// longer stencil) gather in pwd_adj_sample's order.  A source outside its
+// stencil's range holds zeros, which leave a sum as it is.  Same volume: 52
+// -> 38 us, bound by the taps in double of the four rows; keeping them in
+// memory instead would read five floats a sample and row.
+template <int NW>
+__global__ void __launch_bounds__(TB)
+pwd_adj_range(const float *__restrict__ rr, const unsigned char *__restrict__ known, float *__restrict__ gout, Geo g,
+              double *part, const SolverState *st) {
+    constexpr int NA = 2 * NW + 1;
+    __shared__ float pr[4][NA][TB];
+    __shared__ double sh[16];
+    if (st && solver_done(st)) return;
+    const int t = threadIdx.x, H = NW * (g.nparts == 2 ? max(g.nj1, g.nj2) : g.nj1), W = TB - 2 * H;
+    const long per = (g.n + gridDim.x - 1) / gridDim.x;
+    const long k0 = (long)blockIdx.x * per, k1 = min(g.n, k0 + per);
+    double acc = 0.0;
+    for (long c = k0; c < k1; c += W) {
+        const long k = c - H + t;  // this thread's sample, as output and as source
+        float p[4][NA];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {  // part q / 2: the trace before, then the own one
+            if (q / 2 >= g.nparts) continue;
+            const int part_id = q / 2, h = NW * (part_id ? g.nj2 : g.nj1);
+            const long ip = part_id ? (long)g.n1 * g.n2 : g.n1, i = q & 1 ? k : k - ip;
+            const bool in = i >= 0 && i < g.n;
+            const long ic = in ? i : 0;
+            int ix, iy, iz;
+            sample_pos(g, ic, ix, iy, iz);
+            const bool on = in && ix >= h && ix < g.n1 - h && (part_id ? iz < g.n3 - 1 : iy < g.n2 - 1);
+            const float yv = rr[part_id * g.n + ic];
+            float a[NA];
+            apf_pass<NW>(g.slope[part_id][ic], a);
+#pragma unroll
+            for (int j = 0; j < NA; j++) p[q][j] = on ? yv * a[j] : 0.0f;
+        }
+        __syncthreads();  // the last range's gathers are done
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (q / 2 < g.nparts)
+#pragma unroll
+                for (int j = 0; j < NA; j++) pr[q][j][t] = p[q][j];
+        __syncthreads();
+        if (t >= H && t < H + W && k < k1) {
+            float v = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; q += 2) {
+                if (q / 2 >= g.nparts) continue;
+                const int nj = q ? g.nj2 : g.nj1;
+#pragma unroll
+                for (int iw = 2 * NW; iw >= 0; iw--) v = v + pr[q][iw][t - (iw - NW) * nj];
+#pragma unroll
+                for (int iw = 0; iw <= 2 * NW; iw++) v = v - pr[q + 1][iw][t + (iw - NW) * nj];
+            }
+            v = known[k] ? 0.0f : v;
+            gout[k] = v;
+            acc += (double)v * v;
+        }
+    }
+    const double s = block_sum(acc, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
 // partial sums over a vector: sum a*b (stacked into part[k*nblk + b])
 __global__ void __launch_bounds__(TB) dot_kernel(const float *__restrict__ a, const float *__restrict__ b, long n,
                                                  double *part, int slot, int nblk) {
@@ -538,9 +638,28 @@ int pwd_vblocks() {
     return (v == 1 || v == 2 || v == 4) ? v : 2;
 }
 
+// Whether the range kernels run: not with drift, nor for stencils that reach
+// so far along the trace that the adjoint's ranges would overlap by more than
+// a quarter (beyond that the old kernel's 20 separate taps cost no more), nor
+// where SH_PWD_V asks for the kernels of one sum per TB samples.
+bool pwd_ranges(const Geo &g) {
+    const int reach = g.nw * (g.nparts == 2 ? std::max(g.nj1, g.nj2) : g.nj1);
+    return !g.drift && !getenv("SH_PWD_V") && reach <= TB / 8;
+}
+
+// Their blocks over n samples.  The forward measured 40, 38 and 40 us with
+// 1024, 2048 and 4096 blocks at most, the adjoint 46, 42 and 38 (its last
+// wave of blocks is shorter), and the scalar step takes 1 us more for 2048
+// blocks more of the forward's six sums.
+int pwd_range_blocks(long n, int most) { return (int)std::min<long>(ceil_div(n, TB), most); }
+
 template <int NW>
 int pwd_fwd_launch(sh_ctx *ctx, const Geo &g, const float *x, float *y, const float *ss, const float *rr,
                    double *part, int nblk, const float *base, const SolverState *st) {
+    if (pwd_ranges(g)) {
+        hipLaunchKernelGGL((pwd_fwd_range<NW>), dim3(nblk), dim3(TB), 0, ctx->stream, x, y, ss, rr, g, part, base, st);
+        return sh_launch_check(ctx, "pwd_fwd");
+    }
     const int V = pwd_vblocks();
     const dim3 grid(ceil_div(nblk, V));
 #define PF_(D, VV)                                                                                             \
@@ -557,6 +676,10 @@ int pwd_fwd_launch(sh_ctx *ctx, const Geo &g, const float *x, float *y, const fl
 template <int NW>
 int pwd_adj_launch(sh_ctx *ctx, const Geo &g, const float *rr, const unsigned char *known, float *gout, double *part,
                    int nblk, const SolverState *st) {
+    if (pwd_ranges(g)) {
+        hipLaunchKernelGGL((pwd_adj_range<NW>), dim3(nblk), dim3(TB), 0, ctx->stream, rr, known, gout, g, part, st);
+        return sh_launch_check(ctx, "pwd_adj");
+    }
     const int V = pwd_vblocks();
     const dim3 grid(ceil_div(nblk, V));
 #define PA_(D, VV)                                                                                             \
@@ -586,6 +709,9 @@ int soint_solve(sh_ctx *ctx, const Geo &g0, const float *pp, const float *qq, co
     g.d1 = FastDiv((unsigned)g.n1);
     g.d2 = FastDiv((unsigned)g.n2);
     int nbn = ceil_div(n, TB), nby = ceil_div(ny, TB);
+    // blocks of the two operators, whose sums the scalar step adds up
+    const bool ranges = pwd_ranges(g);
+    const int nba = ranges ? pwd_range_blocks(n, 4096) : nbn, nbf = ranges ? pwd_range_blocks(ny, 2048) : nby;
     double *part = nullptr;
     SH_TRY(sh_slot(ctx, SLOT_RED, (size_t)(6 * nby + nbn) * sizeof(double), (void **)&part));
     SolverState *st = nullptr;
@@ -615,8 +741,8 @@ int soint_solve(sh_ctx *ctx, const Geo &g0, const float *pp, const float *qq, co
     // rr = -dd, then rr += A x0 tap by tap (ps_solver 1018-1026); its
     // partial rr.rr starts the solver state
     hipLaunchKernelGGL(neg_kernel, dim3(nby), dim3(TB), 0, ctx->stream, dd, rr, ny);
-    SH_TRY(pwd_fwd_launch<NW>(ctx, g, x, rr, Ss, Ss, part, nby, rr, nullptr));
-    hipLaunchKernelGGL(solver_init, dim3(1), dim3(1024), 0, ctx->stream, part, nby, st, 0);
+    SH_TRY(pwd_fwd_launch<NW>(ctx, g, x, rr, Ss, Ss, part, nbf, rr, nullptr));
+    hipLaunchKernelGGL(solver_init, dim3(1), dim3(1024), 0, ctx->stream, part, nbf, st, 0);
     SH_TRY(sh_launch_check(ctx, "soint init"));
     double *pa = part + (size_t)6 * nby;  // |g|^2 partials of pwd_adj
     // one iteration: g = A^T r (zero where known), A g with the six dots,
@@ -626,15 +752,15 @@ int soint_solve(sh_ctx *ctx, const Geo &g0, const float *pp, const float *qq, co
     auto iteration = [&]() -> int {
         {
             PROF_A(ctx);
-            SH_TRY(pwd_adj_launch<NW>(ctx, g, rr, known, gv, pa, nbn, st));
+            SH_TRY(pwd_adj_launch<NW>(ctx, g, rr, known, gv, pa, nba, st));
             PROF_B(ctx, "pwd_adj", 4.0 * (ny + g.nparts * n + n));
         }
         {
             PROF_A(ctx);
-            SH_TRY(pwd_fwd_launch<NW>(ctx, g, gv, gg, Ss, rr, part, nby, nullptr, st));
+            SH_TRY(pwd_fwd_launch<NW>(ctx, g, gv, gg, Ss, rr, part, nbf, nullptr, st));
             PROF_B(ctx, "pwd_fwd", 4.0 * (n + g.nparts * n + 3 * ny));
         }
-        hipLaunchKernelGGL(cgstep_scalars, dim3(1), dim3(1024), 0, ctx->stream, pa, nbn, part, nby, st, 0);
+        hipLaunchKernelGGL(cgstep_scalars, dim3(1), dim3(1024), 0, ctx->stream, pa, nba, part, nbf, st, 0);
         PROF_A(ctx);
         hipLaunchKernelGGL(cgstep_update, dim3(nby), dim3(TB), 0, ctx->stream, S, gv, x, n, Ss, gg, rr, ny, st);
         PROF_B(ctx, "cgstep_update", 4.0 * (5 * n + 5 * ny));

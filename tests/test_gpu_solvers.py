@@ -205,6 +205,33 @@ def test_pwd_virtual_blocks_identical(ps, monkeypatch):
             assert ia == ib
 
 
+@pytest.mark.parametrize("shape,order,njs", [((8, 2, 2), 1, (1, 1)), ((13, 5, 1), 3, (1, 1)), ((252, 3, 4), 2, (1, 3)),
+                                             ((301, 19, 1), 2, (2, 1)), ((257, 7, 9), 6, (5, 1)),
+                                             ((140, 5, 6), 2, (16, 16)), ((140, 5, 6), 2, (17, 1)),
+                                             ((31, 150, 140), 2, (1, 2)), ((2100, 130, 7), 3, (1, 1))])
+def test_pwd_ranges_equal_single_samples(ps, monkeypatch, shape, order, njs):
+    """soint's operators over ranges of samples (one sum a block, the
+    adjoint's products handed over in LDS) and one sum per 256 samples
+    (SH_PWD_V): traces as long as a range's inner part and off it by some,
+    stencils that reach over a trace's ends and to the rule's edge, more
+    ranges than blocks.  Float operations agree; the order of the double sums
+    may round a scalar to another float: a few 2^-24 an iteration."""
+    d, m, p, q = _case3(shape, 41)
+    if shape[2] == 1:
+        d, m, p = d[:, :, 0], m[:, :, 0], p[:, :, 0]
+
+    def call():
+        if shape[2] == 1:
+            return ps.soint2dc(d, m, p, order=order, njs=list(njs), niter=5, report=True)
+        return ps.soint3dc(d, m, p, q, order=order, njs=list(njs), niter=5, report=True)
+
+    new, it = call()
+    monkeypatch.setenv("SH_PWD_V", "1")
+    old, it0 = call()
+    assert it == it0
+    assert np.abs(new - old).max() <= 5 * 8 * 2.0**-24 * max(np.abs(old).max(), 1.0)
+
+
 @pytest.mark.parametrize("shape,rect,order,masked", [((8, 2), (3, 2), 1, False), ((31, 15), (1, 1), 2, False),
                                                      ((33, 17), (10, 20), 2, True), ((64, 32), (5, 1), 3, False),
                                                      ((130, 70), (1, 9), 2, True), ((515, 257), (10, 20), 2, False),
