@@ -106,81 +106,140 @@ bandpass_traces(float *__restrict__ x, long ntr, int n1, const Butter blo, const
 // trace (butter_pass), in the same order; only the loop nesting changes.
 constexpr int BP_FUSE_MAX = 8;
 struct Stage {
-    int odd, low;
-    float d0, d1, d2;
+    int odd;
+    float c, d0, d1, d2;  // c: the factor of the middle input term, (low ? 1 : -1) times 1 (odd) or 2
 };
 struct Cascade {
     Stage st[BP_FUSE_MAX];
 };
 
 int cascade_of(const Butter &bw, Cascade &c, int ns) {
-    if (bw.nn % 2) c.st[ns++] = Stage{1, bw.low, bw.den[bw.nn / 2][0], 0.0f, bw.den[bw.nn / 2][1]};
-    for (int j = 0; j < bw.nn / 2; j++) c.st[ns++] = Stage{0, bw.low, bw.den[j][0], bw.mid, bw.den[j][1]};
+    if (bw.nn % 2) c.st[ns++] = Stage{1, bw.low ? 1.0f : -1.0f, bw.den[bw.nn / 2][0], 0.0f, bw.den[bw.nn / 2][1]};
+    for (int j = 0; j < bw.nn / 2; j++) c.st[ns++] = Stage{0, bw.low ? 2.0f : -2.0f, bw.den[j][0], bw.mid, bw.den[j][1]};
     return ns;
 }
 
-// 64 traces per block (one wave), staged through LDS in chunks of 64
-// samples: the loads and stores run along the traces (coalesced) and each
-// lane then walks its own trace's column of the tile.  tile[k][r] with row
-// pitch 65 keeps both access patterns free of bank conflicts.
-template <int NS>
-__global__ void __launch_bounds__(64)
-bandpass_fused(float *__restrict__ x, long ntr, int n1, const Cascade c, int back) {
-    __shared__ float tile[64][65];
-    const int t = threadIdx.x;
-    const long tr0 = (long)blockIdx.x * 64;
-    const int nr = (int)min(64L, ntr - tr0);
-    float x0[NS], x1[NS], x2[NS], y1[NS], y2[NS];
+// 64 traces per block, streamed through LDS in chunks of 64 samples: wave 0
+// walks the chunk, one lane per trace, while wave 1 stores the chunk before
+// and has the one after on its way into registers.  tile[k][r] with row
+// pitch 65 keeps the walk (along r) and the memory side (along k, coalesced)
+// free of bank conflicts.  The walk takes about 5 cycles an instruction (one
+// wave a SIMD), 8 instructions a section and sample; with one wave doing
+// both, each chunk waited for its loads besides: 500 samples of 37500 traces,
+// two sections, 128 -> 36 us a pass.  The first pass reads its input where
+// it is.
+//
+// ODD0: the first section is of odd order (its filter's own).  MIX: so may a
+// later one be (both filters in one pass).  A section's sign of the high or
+// low cut is the factor c of its middle term: exact, as 2 x and x are.
+template <int NS, bool ODD0, bool MIX>
+struct Walk {
+    float x1[NS], x2[NS], y1[NS], y2[NS];
+    __device__ void clear() {
 #pragma unroll
-    for (int s = 0; s < NS; s++) x0[s] = x1[s] = x2[s] = y1[s] = y2[s] = 0.0f;
-    const int nch = (n1 + 63) / 64;
-    for (int ci = 0; ci < nch; ci++) {
-        const int k0 = (back ? nch - 1 - ci : ci) * 64;
-        const int cnt = min(64, n1 - k0);
-        if (t < cnt)
-            for (int r = 0; r < nr; r++) tile[t][r] = x[(tr0 + r) * n1 + k0 + t];
-        __syncthreads();
-        if (t < nr) {
-            for (int kk = 0; kk < cnt; kk++) {
-                const int k = back ? cnt - 1 - kk : kk;
-                float v = tile[k][t];
+        for (int s = 0; s < NS; s++) x1[s] = x2[s] = y1[s] = y2[s] = 0.0f;
+    }
+    __device__ float step(const Cascade &c, float v) {
 #pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    const Stage &g = c.st[s];
-                    float y0;
-                    if (g.odd) {
-                        x1[s] = x0[s];
-                        x0[s] = v;
-                        y0 = g.low ? (x0[s] + x1[s] - g.d2 * y1[s]) * g.d0 : (x0[s] - x1[s] - g.d2 * y1[s]) * g.d0;
-                        y1[s] = y0;
-                    } else {
-                        x2[s] = x1[s];
-                        x1[s] = x0[s];
-                        x0[s] = v;
-                        y0 = g.low ? (x0[s] + 2 * x1[s] + x2[s] - g.d1 * y1[s] - g.d2 * y2[s]) * g.d0
-                                   : (x0[s] - 2 * x1[s] + x2[s] - g.d1 * y1[s] - g.d2 * y2[s]) * g.d0;
-                        y2[s] = y1[s];
-                        y1[s] = y0;
-                    }
-                    v = y0;
-                }
-                tile[k][t] = v;
+        for (int s = 0; s < NS; s++) {
+            const Stage &g = c.st[s];
+            const bool odd = s == 0 ? ODD0 : MIX && g.odd;
+            const float t = v + g.c * x1[s];
+            float y0;
+            if (odd) {
+                y0 = (t - g.d2 * y1[s]) * g.d0;
+            } else {
+                y0 = (t + x2[s] - g.d1 * y1[s] - g.d2 * y2[s]) * g.d0;
+                x2[s] = x1[s];
+                y2[s] = y1[s];
             }
+            x1[s] = v;
+            y1[s] = y0;
+            v = y0;
+        }
+        return v;
+    }
+};
+
+constexpr int BP_C = 64;  // traces of a block, samples of a chunk
+
+template <int NS, bool ODD0, bool MIX>
+__global__ void __launch_bounds__(2 * BP_C)
+bandpass_fused(const float *in, float *out, long ntr, int n1, const Cascade c, int back) {
+    __shared__ float tile[2][BP_C][BP_C + 1];
+    const int t = threadIdx.x % BP_C;
+    const bool walks = threadIdx.x < BP_C;
+    const long tr0 = (long)blockIdx.x * BP_C;
+    const int nr = (int)min((long)BP_C, ntr - tr0), nch = (n1 + BP_C - 1) / BP_C;
+    Walk<NS, ODD0, MIX> w;
+    w.clear();
+    float nxt[BP_C];
+    // chunk number ci of the pass: its first sample and its length
+    auto first = [&](int ci) { return (back ? nch - 1 - ci : ci) * BP_C; };
+    auto load = [&](int ci) {
+        const int k = first(ci) + t;
+        const float *p = in + tr0 * n1 + min(k, n1 - 1);
+#pragma unroll
+        for (int r = 0; r < BP_C; r++) nxt[r] = p[(long)min(r, nr - 1) * n1];
+    };
+    auto put = [&](float (*dst)[BP_C + 1]) {
+#pragma unroll
+        for (int r = 0; r < BP_C; r++) dst[t][r] = nxt[r];
+    };
+    auto store = [&](int ci, const float (*src)[BP_C + 1]) {
+        const int k = first(ci) + t;
+        if (k >= n1) return;
+        float *p = out + tr0 * n1 + k;
+#pragma unroll 16
+        for (int r = 0; r < nr; r++) p[(long)r * n1] = src[t][r];
+    };
+    if (!walks) {
+        load(0);
+        put(tile[0]);
+        if (nch > 1) load(1);
+    }
+    __syncthreads();
+    for (int ci = 0; ci < nch; ci++) {
+        float (*cur)[BP_C + 1] = tile[ci & 1], (*other)[BP_C + 1] = tile[~ci & 1];
+        if (walks) {
+            const int cnt = min(BP_C, n1 - first(ci));
+            float *p = &cur[back ? cnt - 1 : 0][t];
+            const int step = back ? -(BP_C + 1) : BP_C + 1;
+            int kk = 0;
+            for (; kk + 8 <= cnt; kk += 8, p += 8 * step) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = p[u * step];
+#pragma unroll
+                for (int u = 0; u < 8; u++) p[u * step] = w.step(c, v[u]);
+            }
+            for (; kk < cnt; kk++, p += step) *p = w.step(c, *p);
+        } else {
+            // the chunk before leaves the other tile, the one after enters it
+            if (ci > 0) store(ci - 1, other);
+            if (ci + 1 < nch) put(other);
+            if (ci + 2 < nch) load(ci + 2);
         }
         __syncthreads();
-        if (t < cnt)
-            for (int r = 0; r < nr; r++) x[(tr0 + r) * n1 + k0 + t] = tile[t][r];
-        __syncthreads();
     }
+    if (!walks) store(nch - 1, tile[(nch - 1) & 1]);
 }
 
-int launch_fused(sh_ctx *ctx, float *x, long ntr, int n1, const Cascade &c, int ns, int back) {
-    const dim3 grid((unsigned)ceil_div(ntr, 64)), block(64);
+int launch_fused(sh_ctx *ctx, const float *in, float *out, long ntr, int n1, const Cascade &c, int ns, int back) {
+    const dim3 grid((unsigned)ceil_div(ntr, BP_C)), block(2 * BP_C);
+    bool mix = false;
+    for (int s = 1; s < ns; s++) mix = mix || c.st[s].odd;
     switch (ns) {
-#define BP_CASE(N) \
-    case N: hipLaunchKernelGGL(bandpass_fused<N>, grid, block, 0, ctx->stream, x, ntr, n1, c, back); break;
+#define BP_K(N, O, M) hipLaunchKernelGGL((bandpass_fused<N, O, M>), grid, block, 0, ctx->stream, in, out, ntr, n1, c, back)
+#define BP_CASE(N)                                               \
+    case N:                                                      \
+        if (mix) { if (c.st[0].odd) BP_K(N, true, true); else BP_K(N, false, true); }   \
+        else if (c.st[0].odd) BP_K(N, true, false);              \
+        else BP_K(N, false, false);                              \
+        break;
         BP_CASE(1) BP_CASE(2) BP_CASE(3) BP_CASE(4) BP_CASE(5) BP_CASE(6) BP_CASE(7) BP_CASE(8)
 #undef BP_CASE
+#undef BP_K
         default: return sh_fail(ctx, SH_EINVAL, "bandpass: %d sections in one pass", ns);
     }
     return sh_launch_check(ctx, "bandpass_fused");
@@ -208,10 +267,16 @@ extern "C" int sh_bandpass(sh_ctx *ctx, const float *in, float *out, int n1, int
     if (flo > eps) butter_init(blo, false, flo, nplo);
     if (fhi < 0.5 - eps) butter_init(bhi, true, fhi, nphi);
     const long ntr = (long)n2 * n3, n = ntr * n1;
-    if (out != in) SH_HIP(ctx, hipMemcpyAsync(out, in, (size_t)n * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
-    if (!blo.on && !bhi.on) return SH_OK;
+    // the fused passes read their input where it is: only what works in place needs the copy
+    auto copy = [&]() -> int {
+        if (out != in)
+            SH_HIP(ctx, hipMemcpyAsync(out, in, (size_t)n * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
+        return SH_OK;
+    };
+    if (!blo.on && !bhi.on) return copy();
     const int slo = blo.on ? blo.nn / 2 + blo.nn % 2 : 0, shi = bhi.on ? bhi.nn / 2 + bhi.nn % 2 : 0;
     if (slo > BP_FUSE_MAX || shi > BP_FUSE_MAX || getenv("SH_BANDPASS_PLAIN")) {
+        SH_TRY(copy());
         hipLaunchKernelGGL(bandpass_traces, dim3((unsigned)ceil_div(ntr, 256)), dim3(256), 0, ctx->stream, out, ntr, n1,
                            blo, bhi, phase);
         return sh_launch_check(ctx, "bandpass_traces");
@@ -225,15 +290,15 @@ extern "C" int sh_bandpass(sh_ctx *ctx, const float *in, float *out, int n1, int
     if (phase && slo + shi <= BP_FUSE_MAX) {
         Cascade both = lo;
         if (bhi.on) cascade_of(bhi, both, slo);
-        return launch_fused(ctx, out, ntr, n1, both, slo + shi, 0);
+        return launch_fused(ctx, in, out, ntr, n1, both, slo + shi, 0);
     }
     if (blo.on) {
-        SH_TRY(launch_fused(ctx, out, ntr, n1, lo, slo, 0));
-        if (!phase) SH_TRY(launch_fused(ctx, out, ntr, n1, lo, slo, 1));
+        SH_TRY(launch_fused(ctx, in, out, ntr, n1, lo, slo, 0));
+        if (!phase) SH_TRY(launch_fused(ctx, out, out, ntr, n1, lo, slo, 1));
     }
     if (bhi.on) {
-        SH_TRY(launch_fused(ctx, out, ntr, n1, hi, shi, 0));
-        if (!phase) SH_TRY(launch_fused(ctx, out, ntr, n1, hi, shi, 1));
+        SH_TRY(launch_fused(ctx, blo.on ? out : in, out, ntr, n1, hi, shi, 0));
+        if (!phase) SH_TRY(launch_fused(ctx, out, out, ntr, n1, hi, shi, 1));
     }
     return SH_OK;
 }
