@@ -5,7 +5,7 @@ HERE="$(cd "$(dirname "$0")" && pwd)"
 OUT="$HERE/../libseistr_hip.so"
 HIPCC=${HIPCC:-/opt/rocm/bin/hipcc}
 JOBS=${JOBS:-8}
-SRCS="common dip dip2"
+SRCS="common dip dip2 smooth"
 [ -f "$HERE/spray.hip" ] && SRCS="$SRCS spray"
 [ -f "$HERE/chain2.hip" ] && SRCS="$SRCS chain2"
 [ -f "$HERE/interp.hip" ] && SRCS="$SRCS interp"

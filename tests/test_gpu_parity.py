@@ -314,6 +314,45 @@ def test_bandpassc_bit_exact(ps, shape, monkeypatch):
         bandpass.bandpass_device(d, shape, 0.004, 5.0, 40.0, 300, 6, 1)
 
 
+@pytest.mark.parametrize("n,other,nb", [(2, 130, 2), (3, 67, 9), (179, 65, 5), (180, 63, 5), (362, 33, 5), (363, 31, 5),
+                                        (16, 257, 8), (953, 17, 5), (954, 15, 5), (1810, 9, 5), (1811, 3, 5),
+                                        (3266, 5, 5), (3267, 5, 5), (40, 129, 40), (40, 129, 41), (33, 64, 700)])
+def test_smoothc_resident_lines_bit_exact(ps, n, other, nb):
+    """Lines of each length that changes how many a block holds in LDS, and
+    one more (3266 is the longest held); ragged numbers of lines; radii up to,
+    at and beyond the axis; the lines along each of the axes."""
+    from oracle import oracle as O
+    from pyseistr_amd import smooth
+    rng = np.random.default_rng(n + nb)
+    for ax, shape in enumerate([(n, other, 1), (other, n, 2), (7, other, n)]):
+        if n * other > 20000 and ax == 2:
+            continue
+        x = rng.standard_normal(int(np.prod(shape))).astype(np.float32)
+        rect = tuple(nb if k == ax else 1 for k in range(3))
+        for adj in (0, 1):
+            for diff, box in (((0, 0, 0), (0, 0, 0)), ((1, 1, 1), (0, 0, 0)), ((0, 0, 0), (1, 1, 1))):
+                got = smooth.smooth_device(_dev(x), shape, rect, diff, box, 1, adj).cpu().numpy()
+                exp = O.smoothc(x, shape, rect, diff, box, 1, adj)
+                assert np.array_equal(got.view(np.uint32), exp.view(np.uint32)), (ax, adj, diff, box)
+
+
+@pytest.mark.parametrize("n1,ntr", [(1, 64), (7, 1), (63, 65), (64, 63), (65, 128), (127, 3), (128, 129), (129, 64), (200, 2)])
+def test_bandpassc_chunk_edges_bit_exact(ps, n1, ntr):
+    """Chunks of 64 samples and blocks of 64 traces, one off either way, with
+    1 to 8 sections in a pass, the odd one first, later and absent; the input
+    is left as it was."""
+    from oracle import oracle as O
+    from pyseistr_amd import bandpass
+    x = np.random.default_rng(n1 + ntr).standard_normal(n1 * ntr).astype(np.float32)
+    d = _dev(x)
+    for nplo, nphi in [(1, 1), (2, 3), (3, 2), (4, 4), (5, 7), (8, 8), (7, 7), (15, 16), (12, 13)]:
+        for phase in (0, 1):
+            got = bandpass.bandpass_device(d, (n1, ntr, 1), 0.004, 6.0, 60.0, nplo, nphi, phase).cpu().numpy()
+            exp = O.bandpass(x, (n1, ntr, 1), 0.004, 6.0, 60.0, nplo, nphi, phase)
+            assert np.array_equal(got.view(np.uint32), exp.view(np.uint32)), (nplo, nphi, phase)
+    assert np.array_equal(d.cpu().numpy(), x)
+
+
 def test_smoothc_bandpassc_full_size_bit_exact(ps):
     """At the benchmark's 512 x 256 x 256: smoothc (rect 5,5,5, and a
     derivative / box mix) and bandpassc (zero and minimum phase) bit for bit
