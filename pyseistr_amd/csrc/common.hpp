@@ -46,6 +46,7 @@ struct sh_ctx {
     // FFT plans of the FK dip filter for the last size it ran on (owned;
     // the deleter destroys them)
     std::shared_ptr<void> fk;
+    std::shared_ptr<void> fk_tables;
     // SH_FLAG_* of the public entry points (sh_ctx_set_flags)
     int flags = 0;
     // brackets of a dip call's device time (sh_dip_report.elapsed_ms)

@@ -56,6 +56,28 @@ def test_one_dimensional_transforms_agree(fk, monkeypatch, shape):
     assert _rel(one, ref) <= TOL and _rel(two, ref) <= TOL
 
 
+@pytest.mark.parametrize("n1", [65, 128, 129, 400, 513, 2048, 2500, 4097, 9001, 16384])
+@pytest.mark.parametrize("n2", [33, 64, 90, 257, 600, 2000])
+def test_transform_lengths(fk, n1, n2):
+    """Every length of the three-kernel path along time (128 to 16384, the
+    odd and even ends of a trace) against each along space (64 to 2048, with
+    and without padding; 4096 is in the section above): the rounding of its
+    log2(n) additions a value stays far below the bar."""
+    if n1 * n2 > 10_000_000:
+        n2 = n2 // 16 + 33
+    d = np.random.default_rng(n1 + n2).standard_normal((n1, n2))
+    for w in (0.03, 0.4):
+        got, ref = fk.fkdip(d, w), F.fkdip(d, w)
+        assert _rel(got, ref) <= TOL
+
+
+def test_lengths_left_to_the_library(fk):
+    """One step beyond the three kernels' range on each side."""
+    for shape in [(64, 100), (16385, 40), (200, 32), (130, 4097)]:
+        d = np.random.default_rng(shape[0]).standard_normal(shape)
+        assert _rel(fk.fkdip(d, 0.1), F.fkdip(d, 0.1)) <= TOL
+
+
 def test_repeated_and_resized_calls(fk):
     # the plans are cached per size: alternate sizes and repeat
     rng = np.random.default_rng(3)
