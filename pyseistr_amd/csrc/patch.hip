@@ -21,9 +21,11 @@ struct PGeo {
 // one per plane position and the block's patch-number split.
 // Blocks are dealt to the eight XCDs in turn; block b takes patch
 // (b % 8) * per + b / 8, so each XCD works through a contiguous run of patch
-// numbers and the overlapping neighbours share its L2.
+// numbers and the overlapping neighbours share its L2.  Bound by writing the
+// patches; a plane's eight samples in flight instead of one: the section
+// below 175 -> 150 us (non-temporal stores 161).
 __global__ void patch_cut(const double *__restrict__ in, double *__restrict__ X, PGeo g, long L, int npatch,
-                          int per) {
+                          int per, FastDiv d1) {
     const int pid = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
     if (pid >= npatch) return;
     const int p3 = pid % g.P[2], p2 = (pid / g.P[2]) % g.P[1], p1 = pid / (g.P[1] * g.P[2]);
@@ -32,6 +34,27 @@ __global__ void patch_cut(const double *__restrict__ in, double *__restrict__ X,
     const long n12 = (long)g.n[0] * g.n[1];
     const int m3 = min(l3, g.n[2] - b3);  // axis-3 samples inside the volume (may be <= 0)
     double *row = X + (long)pid * L;
+    if (l3 == 1) {  // a plane: eight of the thread's samples in flight
+        constexpr int U = 8;
+        const double *src = in + n12 * min(b3, g.n[2] - 1);
+        for (long q0 = threadIdx.x; q0 < l12; q0 += U * blockDim.x) {
+            double v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int q = (int)min(q0 + u * (long)blockDim.x, (long)l12 - 1);
+                const int e2 = (int)d1.div((unsigned)q), i1 = b1 + (q - e2 * l1), i2 = b2 + e2;
+                const bool ok = i1 < g.n[0] && i2 < g.n[1] && m3 > 0;
+                const double t = src[ok ? i1 + (long)g.n[0] * i2 : 0];
+                v[u] = ok ? t : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const long q = q0 + u * (long)blockDim.x;
+                if (q < l12) row[q] = v[u];
+            }
+        }
+        return;
+    }
     for (int q = threadIdx.x; q < l12; q += blockDim.x) {
         const int i1 = b1 + q % l1, i2 = b2 + q / l1;
         const bool ok = i1 < g.n[0] && i2 < g.n[1];
@@ -59,7 +82,11 @@ __device__ inline void covering(int i, int l, int s, int P, int &lo, int &hi) {
 
 // One block per (i2, i3) column of the output, threads along i1.  Every
 // sample adds its covering patches in patch order (p1, then p2, then p3),
-// the order in which the reference accumulates them.
+// the order in which the reference accumulates them.  Bound by reading X,
+// each value once: the loads are non-temporal, of four samples at a time.
+// 6000 x 2500 in patches of 256 x 128, half overlapping (0.48 GB of patches):
+// 167 us with one load in flight, 137 with four, 115 non-temporal (the copy's
+// rate takes 128 us).
 __global__ void patch_paste(const double *__restrict__ X, double *__restrict__ out, PGeo g, long L) {
     const int c = blockIdx.x;
     const int i2 = c % g.n[1], i3 = c / g.n[1];
@@ -67,22 +94,40 @@ __global__ void patch_paste(const double *__restrict__ X, double *__restrict__ o
     covering(i2, g.l[1], g.s[1], g.P[1], lo2, hi2);
     covering(i3, g.l[2], g.s[2], g.P[2], lo3, hi3);
     const long l1 = g.l[0], l12 = (long)g.l[0] * g.l[1];
-    for (int i1 = threadIdx.x; i1 < g.n[0]; i1 += blockDim.x) {
-        int lo1, hi1;
-        covering(i1, g.l[0], g.s[0], g.P[0], lo1, hi1);
-        double acc = 0.0, cnt = 0.0;
-        for (int p1 = lo1; p1 <= hi1; p1++) {
-            const long e1 = i1 - p1 * g.s[0];
-            for (int p2 = lo2; p2 <= hi2; p2++) {
-                const long id0 = ((long)p1 * g.P[1] + p2) * g.P[2];
-                const long e12 = e1 + l1 * (i2 - p2 * g.s[1]);
-                for (int p3 = lo3; p3 <= hi3; p3++) {
-                    acc += X[(id0 + p3) * L + e12 + l12 * (i3 - p3 * g.s[2])];
-                    cnt += 1.0;
-                }
-            }
+    constexpr int U = 4;  // samples of a thread whose loads are in flight together
+    for (long i0 = threadIdx.x; i0 < g.n[0]; i0 += U * blockDim.x) {
+        int lo1[U], hi1[U], most = 0;
+        double acc[U], cnt[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            covering((int)min(i0 + u * (long)blockDim.x, g.n[0] - 1L), g.l[0], g.s[0], g.P[0], lo1[u], hi1[u]);
+            most = max(most, hi1[u] - lo1[u] + 1);
+            acc[u] = cnt[u] = 0.0;
         }
-        out[(long)c * g.n[0] + i1] = acc / cnt;
+        for (int k = 0; k < most; k++)
+            for (int p2 = lo2; p2 <= hi2; p2++)
+                for (int p3 = lo3; p3 <= hi3; p3++) {
+                    const long e23 = l1 * (i2 - p2 * g.s[1]) + l12 * (i3 - p3 * g.s[2]);
+                    double v[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const int i1 = (int)min(i0 + u * (long)blockDim.x, g.n[0] - 1L), p1 = lo1[u] + k;
+                        const bool on = p1 <= hi1[u];
+                        const long id = ((long)p1 * g.P[1] + p2) * g.P[2] + p3;
+                        v[u] = __builtin_nontemporal_load(X + (on ? id * L + (i1 - p1 * g.s[0]) + e23 : 0));
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        if (lo1[u] + k <= hi1[u]) {
+                            acc[u] += v[u];
+                            cnt[u] += 1.0;
+                        }
+                }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const long i1 = i0 + u * (long)blockDim.x;
+            if (i1 < g.n[0]) out[(long)c * g.n[0] + i1] = acc[u] / cnt[u];
+        }
     }
 }
 
@@ -130,7 +175,8 @@ extern "C" int sh_patch(sh_ctx *ctx, const double *in, double *X, int n1, int n2
     SH_TRY(geometry(ctx, n1, n2, n3, l1, l2, l3, s1, s2, s3, g, np, L));
     const int tpb = (int)std::min<long>(256, ceil_div((long)l1 * l2, 64) * 64);
     const int per = (int)ceil_div(np, 8);
-    hipLaunchKernelGGL(patch_cut, dim3((unsigned)(8L * per)), dim3(tpb), 0, ctx->stream, in, X, g, L, (int)np, per);
+    hipLaunchKernelGGL(patch_cut, dim3((unsigned)(8L * per)), dim3(tpb), 0, ctx->stream, in, X, g, L, (int)np, per,
+                       FastDiv((unsigned)l1));
     return sh_launch_check(ctx, "patch_cut");
 }
 

@@ -43,6 +43,19 @@ def test_patch2d_bit_exact(pm, n, l, s, dt):
                           equal_nan=True)
 
 
+@pytest.mark.parametrize("n,l,s", [((1023, 20), (1023, 1), (3, 1)), ((1025, 12), (100, 12), (7, 5)), ((2050, 9), (1024, 2), (512, 1)),
+                                   ((300, 40), (41, 50), (41, 20)), ((5000, 3), (2049, 3), (683, 2))])
+def test_batches_of_a_thread_bit_exact(pm, n, l, s):
+    """Traces and planes around the samples a block's threads hold at a time
+    (1024 and 2048), one off either way, and numbers of covering patches that
+    differ among a thread's samples."""
+    A = np.random.default_rng(n[0]).standard_normal(n)
+    X = pm.patch2d(A, *l, *s)
+    assert np.array_equal(X, P.cut(A, l, s))
+    Y = np.random.default_rng(n[1]).standard_normal(X.shape)
+    assert np.array_equal(pm.patch2d_inv(Y, *n, *l, *s), P.paste(Y, n, l, s), equal_nan=True)
+
+
 @pytest.mark.parametrize("pad", list(itertools.product([0, 1], repeat=3)))
 def test_patch3d_every_padding_case(pm, pad):
     # l = (6, 4, 4), s = (3, 2, 2): n fits exactly when (n - l) % s == 0
