@@ -249,6 +249,12 @@ pwd_adj(const float *__restrict__ rr, const unsigned char *__restrict__ known,
     }
 }
 
+// samples of a block's range: as many passes of w as share them out
+__device__ inline long range_of(long n, int w) {
+    const long passes = (n + w - 1) / w;
+    return (passes + gridDim.x - 1) / gridDim.x * w;
+}
+
 // The operators without drift.  Each block runs a contiguous range of
 // samples and sums once at its end: with a sum per 256 samples the wave sums
 // of the six dots were most of pwd_fwd's instructions, and adding up 23
@@ -263,7 +269,7 @@ pwd_fwd_range(const float *__restrict__ x, float *__restrict__ y, const float *_
               const float *__restrict__ rr, Geo g, double *part, const float *base, const SolverState *st) {
     __shared__ double sh[16 * 6];
     if (st && solver_done(st)) return;
-    const long ny = g.n * g.nparts, per = (ny + gridDim.x - 1) / gridDim.x;
+    const long ny = g.n * g.nparts, per = range_of(ny, TB);
     const long i0 = (long)blockIdx.x * per, i1 = min(ny, i0 + per);
     double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     for (long c = i0; c < i1; c += TB) {
@@ -300,7 +306,7 @@ pwd_adj_range(const float *__restrict__ rr, const unsigned char *__restrict__ kn
     __shared__ double sh[16];
     if (st && solver_done(st)) return;
     const int t = threadIdx.x, H = NW * (g.nparts == 2 ? max(g.nj1, g.nj2) : g.nj1), W = TB - 2 * H;
-    const long per = (g.n + gridDim.x - 1) / gridDim.x;
+    const long per = range_of(g.n, W);
     const long k0 = (long)blockIdx.x * per, k1 = min(g.n, k0 + per);
     double acc = 0.0;
     for (long c = k0; c < k1; c += W) {
@@ -638,20 +644,23 @@ int pwd_vblocks() {
     return (v == 1 || v == 2 || v == 4) ? v : 2;
 }
 
+// How far the adjoint's longer stencil reaches along the trace, to each side.
+int pwd_reach(const Geo &g) { return g.nw * (g.nparts == 2 ? std::max(g.nj1, g.nj2) : g.nj1); }
+
 // Whether the range kernels run: not with drift, nor for stencils that reach
 // so far along the trace that the adjoint's ranges would overlap by more than
 // a quarter (beyond that the old kernel's 20 separate taps cost no more), nor
 // where SH_PWD_V asks for the kernels of one sum per TB samples.
-bool pwd_ranges(const Geo &g) {
-    const int reach = g.nw * (g.nparts == 2 ? std::max(g.nj1, g.nj2) : g.nj1);
-    return !g.drift && !getenv("SH_PWD_V") && reach <= TB / 8;
-}
+bool pwd_ranges(const Geo &g) { return !g.drift && !getenv("SH_PWD_V") && pwd_reach(g) <= TB / 8; }
 
-// Their blocks over n samples.  The forward measured 40, 38 and 40 us with
-// 1024, 2048 and 4096 blocks at most, the adjoint 46, 42 and 38 (its last
-// wave of blocks is shorter), and the scalar step takes 1 us more for 2048
-// blocks more of the forward's six sums.
-int pwd_range_blocks(long n, int most) { return (int)std::min<long>(ceil_div(n, TB), most); }
+// Their blocks over n samples in passes of w.  The forward measured 40, 38
+// and 40 us with 1024, 2048 and 4096 blocks at most, the adjoint 46, 42 and
+// 38 (its last wave of blocks is shorter), and the scalar step takes 1 us
+// more for 2048 blocks more of the forward's six sums.
+int pwd_range_blocks(long n, int w, int most) {
+    const int passes = ceil_div(n, w);
+    return ceil_div(passes, ceil_div(passes, most));
+}
 
 template <int NW>
 int pwd_fwd_launch(sh_ctx *ctx, const Geo &g, const float *x, float *y, const float *ss, const float *rr,
@@ -711,9 +720,10 @@ int soint_solve(sh_ctx *ctx, const Geo &g0, const float *pp, const float *qq, co
     int nbn = ceil_div(n, TB), nby = ceil_div(ny, TB);
     // blocks of the two operators, whose sums the scalar step adds up
     const bool ranges = pwd_ranges(g);
-    const int nba = ranges ? pwd_range_blocks(n, 4096) : nbn, nbf = ranges ? pwd_range_blocks(ny, 2048) : nby;
+    const int nba = ranges ? pwd_range_blocks(n, TB - 2 * pwd_reach(g), 4096) : nbn;
+    const int nbf = ranges ? pwd_range_blocks(ny, TB, 2048) : nby;
     double *part = nullptr;
-    SH_TRY(sh_slot(ctx, SLOT_RED, (size_t)(6 * nby + nbn) * sizeof(double), (void **)&part));
+    SH_TRY(sh_slot(ctx, SLOT_RED, (size_t)(6 * nby + std::max(nbn, nba)) * sizeof(double), (void **)&part));
     SolverState *st = nullptr;
     SH_TRY(sh_slot(ctx, SLOT_SCAL, sizeof(SolverState), (void **)&st));
     int *ids = nullptr;
