@@ -238,6 +238,31 @@ __device__ inline void sm_weights(float *wts, int nb) {
         wts[k] = (float)((double)(nb - k) / ((double)nb * nb));
 }
 
+// Triangle stencils of four neighbouring outputs: c points at the first
+// one's sample, st is the stride.  Each output is w[0] c[0] + sum_k w[k]
+// (c[-k] + c[k]), k ascending; two loads a k serve all four.
+__device__ inline void tri4(const float *c, int st, const float *w, int h, float *o) {
+    float l[4], r[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        l[j] = r[j] = c[j * st];
+        o[j] = w[0] * l[j];
+    }
+#pragma unroll 4
+    for (int k = 1; k <= h; k++) {
+        // l[j] = c[j - k], r[j] = c[j + k]
+#pragma unroll
+        for (int j = 3; j > 0; j--) l[j] = l[j - 1];
+        l[0] = c[-k * st];
+#pragma unroll
+        for (int j = 0; j < 3; j++) r[j] = r[j + 1];
+        r[3] = c[(3 + k) * st];
+        const float wk = w[k];
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[j] += wk * (l[j] + r[j]);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Per-sample PWD stencil (allpass1 / allpass2, dip_cfuns.c:1135-1200,
 // 1399-1465) at flat index i, with ip the offset of the next trace along the

@@ -80,6 +80,50 @@ def test_dip2d_batched_matches_per_patch(env, tile):
     assert same == len(pats)
 
 
+@pytest.mark.parametrize("tile,rect", [(2, (1, 1, 1)), (2, (25, 2, 1)), (1, (4, 40, 1)), (4, (90, 3, 1)), (5, (1, 20, 1)),
+                                       (3, (30, 10, 1)), (0, (45, 33, 1)), (2, (32, 32, 1)), (2, (39, 33, 1))])
+def test_batched_smoothing_edges(env, tile, rect):
+    """Patches of a sample or a trace more or less than a tile, down to two
+    traces and fewer samples than the stencil or the smoothing reach, radii
+    from none to the largest a tile takes (its staging then needs more than
+    64 KB of LDS): as the sections one by one, to the bar above."""
+    from pyseistr_amd import dip
+    batch, _ = env
+    rng = np.random.default_rng(rect[0])
+    pats = [rng.standard_normal(sh).astype(np.float32) for sh in
+            [(64, 16), (65, 17), (63, 15), (3, 40), (129, 2), (200, 33), (3, 2), (257, 9)]]
+    b = batch.Batch(pats)
+    got, rec = batch.dip2d_batched(b, niter=2, liter=4, order=2, rect=rect, tile=tile, report=True)
+    for x, g in zip(pats, b.split(got)):
+        ref = dip.dip2dc(x, niter=2, liter=4, order=2, rect=list(rect), verb=0)
+        assert np.abs(g - ref).max() <= 1e-4
+
+
+def test_batch_workspace_reuse_and_gaps(env):
+    """The fields of a batch are not cleared: a batch run after one of other
+    patches gives the bits it gives first, and the slopes between patches
+    with a gap stay zero."""
+    import torch
+    batch, pats = env
+    b, big = batch.Batch(pats[:2]), batch.Batch(pats)
+    first = b.split(batch.dip2d_batched(b, niter=3, liter=6))
+    med = b.split(batch.somf2d_batched(b, batch.Batch(first).data, ns=5))
+    batch.somf2d_batched(big, batch.dip2d_batched(big, niter=2, liter=6) * float("nan"), ns=5)
+    again = b.split(batch.dip2d_batched(b, niter=3, liter=6))
+    med2 = b.split(batch.somf2d_batched(b, batch.Batch(again).data, ns=5))
+    for u, v, m, w in zip(first, again, med, med2):
+        assert np.array_equal(_bits(u), _bits(v)) and np.array_equal(_bits(m), _bits(w))
+    gap = 77
+    g = batch.Batch(shapes=b.shapes)
+    g.offs, g.ntot = b.offs + np.arange(2) * gap, b.ntot + gap
+    cut = int(b.offs[1])
+    g.data = torch.cat([b.data[:cut], torch.full((gap,), 3.0, device="cuda"), b.data[cut:]])
+    flat = batch.dip2d_batched(g, niter=3, liter=6).cpu().numpy()
+    assert not flat[cut:cut + gap].any()
+    whole = np.concatenate([flat[:cut], flat[cut + gap:]])
+    assert np.array_equal(_bits(whole), _bits(np.concatenate([u.ravel(order="F") for u in first])))
+
+
 def test_dip2d_batched_against_oracle(env):
     from oracle import oracle as O
     batch, pats = env
