@@ -345,8 +345,10 @@ bsmooth2(const float *__restrict__ in, int r1, int r2, CgArgs A, const BPatch *_
 // (which = 1), then the patch's scalar step.  One wave per patch.
 __global__ void __launch_bounds__(64)
 bfinalize(const double *part, int stride, int K, int which, const BPatch *__restrict__ P, DipScal *sc, int mode,
-          int it, float tol, int k_ls) {
+          int it, float tol) {
     const int pi = blockIdx.x, lane = threadIdx.x;
+    // a solve or line search that is over: dip_scalar_step changes nothing
+    if (((mode == F_GN || mode == F_BETA) && sc[pi].cg_done) || (mode == F_LS7 && sc[pi].accepted)) return;
     const BPatch q = P[pi];
     const int b0 = which == 0 ? q.blk0 : q.tile0, nb = which == 0 ? q.nblk : q.ntile;
     double tot[LS_SUMS] = {};
@@ -355,7 +357,7 @@ bfinalize(const double *part, int stride, int K, int which, const BPatch *__rest
         for (int b = lane; b < nb; b += 64) s += part[(size_t)k * stride + b0 + b];
         tot[k] = wave_sum(s);
     }
-    if (lane == 0) dip_scalar_step(sc + pi, tot, mode, it, (long)q.n1 * q.n2, tol, k_ls);
+    if (lane == 0) dip_scalar_step(sc + pi, tot, mode, it, (long)q.n1 * q.n2, tol);
 }
 
 __global__ void bfill(float *__restrict__ y, float v, long n) {
@@ -428,7 +430,7 @@ int bsmooth(sh_ctx *ctx, int cfg, const BatchTables &T, int r1, int r2, const fl
 int bfin(sh_ctx *ctx, const BatchTables &T, BWork &W, int K, int which, int mode, int it) {
     int stride = which == 0 ? T.nblk : T.ntile;
     hipLaunchKernelGGL(bfinalize, dim3(T.np), dim3(64), 0, ctx->stream, W.part, stride, K, which, T.P, W.sc, mode,
-                       it, 1.e-6f, 0);
+                       it, 1.e-6f);
     return sh_launch_check(ctx, "bfinalize");
 }
 

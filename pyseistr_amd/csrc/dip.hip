@@ -25,9 +25,11 @@ using namespace dipcore;
 // Reductions + scalar logic, one block of 1024 threads.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(1024) dip_finalize(const double *part, int nblk, int K, DipScal *sc,
-                                                     int mode, int it, long n, float tol, int k_ls) {
+                                                     int mode, int it, long n, float tol) {
     __shared__ double sh[16];
-    __shared__ double tot[4];
+    __shared__ double tot[8];
+    // a solve or line search that is over: dip_scalar_step changes nothing
+    if (((mode == F_GN || mode == F_BETA) && sc->cg_done) || (mode == F_LS7 && sc->accepted)) return;
     for (int k = 0; k < K; k++) {
         double s = 0.0;
         for (int i = threadIdx.x; i < nblk; i += blockDim.x) s += part[(size_t)k * nblk + i];
@@ -36,7 +38,7 @@ __global__ void __launch_bounds__(1024) dip_finalize(const double *part, int nbl
         __syncthreads();
     }
     if (threadIdx.x != 0) return;
-    dip_scalar_step(sc, tot, mode, it, n, tol, k_ls);
+    dip_scalar_step(sc, tot, mode, it, n, tol);
 }
 
 // ---------------------------------------------------------------------------
@@ -46,6 +48,25 @@ __global__ void __launch_bounds__(1024) dip_finalize(const double *part, int nbl
 //         scale by 1/hypot(den, 1) (dip_cfuns.c:1656-1663, 802-808), sum den^2
 // MODE 2: line-search trial p = clip(p0 + lam dp), u2 = C(p) x, sum u2^2
 // ---------------------------------------------------------------------------
+// whether the stencil at sample i lies inside (fast: multiply-high division)
+template <int NW>
+__device__ inline bool pwd_inside(long i, int n1, int n2, int n3, int axis, bool fast, const FastDiv &f1,
+                                  const FastDiv &f2) {
+    int i1, i2, i3;
+    if (fast) {
+        const unsigned r = f1.div((unsigned)i), q = f2.div(r);
+        i1 = (int)((unsigned)i - r * (unsigned)n1);
+        i2 = (int)(r - q * (unsigned)n2);
+        i3 = (int)q;
+    } else {
+        i1 = (int)(i % n1);
+        const long r = i / n1;
+        i2 = (int)(r % n2);
+        i3 = (int)(r / n2);
+    }
+    return i1 >= NW && i1 < n1 - NW && (axis == 2 ? i2 < n2 - 1 : i3 < n3 - 1);
+}
+
 template <int NW, int MODE>
 __global__ void __launch_bounds__(256)
 pwd_kernel(const float *__restrict__ x, const float *__restrict__ p, const float *__restrict__ dp,
@@ -63,23 +84,75 @@ pwd_kernel(const float *__restrict__ x, const float *__restrict__ p, const float
     const long i0 = (long)blockIdx.x * chunk, i1e = min(n, i0 + chunk);
     const bool fast = n < (1L << 31);  // multiply-high division (no long division per sample)
     for (long i = i0 + threadIdx.x; i < i1e; i += blockDim.x) {
-        int i1, i2, i3;
-        if (fast) {
-            const unsigned r = f1.div((unsigned)i), q = f2.div(r);
-            i1 = (int)((unsigned)i - r * (unsigned)n1);
-            i2 = (int)(r - q * (unsigned)n2);
-            i3 = (int)q;
-        } else {
-            i1 = (int)(i % n1);
-            const long r = i / n1;
-            i2 = (int)(r % n2);
-            i3 = (int)(r / n2);
-        }
-        bool valid = i1 >= NW && i1 < n1 - NW && (axis == 2 ? i2 < n2 - 1 : i3 < n3 - 1);
+        const bool valid = pwd_inside<NW>(i, n1, n2, n3, axis, fast, f1, f2);
         acc += pwd_sample<NW, MODE>(x, p, dp, lam, pmin, pmax, pout, u1, u2, mask && mask[i], i, ip, valid);
     }
     double t = block_sum(acc, sh);
     if (threadIdx.x == 0) part[blockIdx.x] = t;
+}
+
+// The seven halved steps of a line search that refused the full one: their
+// residuals' sums from one read of the data (pwd_sample<NW, 2>'s operations).
+// The eight trials were sixteen launches an iteration, most of them no-ops;
+// the full step, these sums and the chosen step are five.
+constexpr int LS_SUMS = 7;
+
+template <int NW>
+__global__ void __launch_bounds__(256)
+pwd_halved(const float *__restrict__ x, const float *__restrict__ p, const float *__restrict__ dp, float pmin,
+           float pmax, int n1, int n2, int n3, int axis, double *part, const DipScal *sc, FastDiv f1, FastDiv f2) {
+    if (sc->accepted) return;
+    __shared__ double sh[16 * LS_SUMS];
+    const long n = (long)n1 * n2 * n3, ip = (axis == 2) ? n1 : (long)n1 * n2;
+    const bool fast = n < (1L << 31);
+    double acc[LS_SUMS];
+#pragma unroll
+    for (int k = 0; k < LS_SUMS; k++) acc[k] = 0.0;
+    const long chunk = (n + gridDim.x - 1) / gridDim.x;
+    const long i0 = (long)blockIdx.x * chunk, i1e = min(n, i0 + chunk);
+    for (long i = i0 + threadIdx.x; i < i1e; i += blockDim.x) {
+        if (!pwd_inside<NW>(i, n1, n2, n3, axis, fast, f1, f2)) continue;
+        float df[2 * NW + 1];
+#pragma unroll
+        for (int iw = 0; iw <= 2 * NW; iw++) df[iw] = x[i + iw - NW + ip] - x[i - iw + NW];
+        const float p0 = p[i], d = dp[i];
+        float lam = 0.5f;
+#pragma unroll
+        for (int k = 0; k < LS_SUMS; k++) {
+            float pv = p0 + lam * d;
+            if (pv < pmin) pv = pmin;
+            if (pv > pmax) pv = pmax;
+            float a[2 * NW + 1], y = 0.0f;
+            apf_pass<NW>(pv, a);
+#pragma unroll
+            for (int iw = 0; iw <= 2 * NW; iw++) y += df[iw] * a[iw];
+            acc[k] += (double)y * y;
+            lam *= 0.5f;
+        }
+    }
+    block_sum_multi<LS_SUMS>(acc, sh);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < LS_SUMS; k++) part[(size_t)k * gridDim.x + blockIdx.x] = acc[k];
+}
+
+// the step that was kept (the last one if none was accepted), where it is not
+// the full one
+template <int NW>
+__global__ void __launch_bounds__(256)
+pwd_chosen(const float *__restrict__ x, const float *__restrict__ p, const float *__restrict__ dp, float pmin,
+           float pmax, float *__restrict__ pout, float *__restrict__ u2, int n1, int n2, int n3, int axis,
+           const DipScal *sc, FastDiv f1, FastDiv f2) {
+    const int k = min(sc->ls_k, 7);
+    if (k == 0) return;
+    const long n = (long)n1 * n2 * n3, ip = (axis == 2) ? n1 : (long)n1 * n2;
+    const bool fast = n < (1L << 31);
+    const float lam = ldexpf(1.0f, -k);
+    const long chunk = (n + gridDim.x - 1) / gridDim.x;
+    const long i0 = (long)blockIdx.x * chunk, i1e = min(n, i0 + chunk);
+    for (long i = i0 + threadIdx.x; i < i1e; i += blockDim.x)
+        (void)pwd_sample<NW, 2>(x, p, dp, lam, pmin, pmax, pout, nullptr, u2, false, i, ip,
+                                pwd_inside<NW>(i, n1, n2, n3, axis, fast, f1, f2));
 }
 
 // CG start (ps_divne tail + ps_conjgrad head, dip_cfuns.c:819-826, 284-303):
@@ -814,9 +887,9 @@ int smooth_apply(sh_ctx *ctx, const DipGeom &g, const SmoothPlan &sp, const floa
     return SH_OK;
 }
 
-int finalize(sh_ctx *ctx, DipWork &W, int nblk, int K, int mode, int it, long n, int k_ls = 0) {
+int finalize(sh_ctx *ctx, DipWork &W, int nblk, int K, int mode, int it, long n) {
     hipLaunchKernelGGL(dip_finalize, dim3(1), dim3(1024), 0, ctx->stream, W.part, nblk, K, W.sc, mode, it, n,
-                       1.e-6f, k_ls);
+                       1.e-6f);
     return sh_launch_check(ctx, "dip_finalize");
 }
 
@@ -871,12 +944,17 @@ int dip_direction(sh_ctx *ctx, const DipGeom &g, const SmoothPlan &plan, int axi
         hipLaunchKernelGGL(cg_result_kernel, dim3(nb_pw), dim3(256), 0, ctx->stream, W.xa, W.xb, W.sx, W.dp, n,
                            W.sc);
         SH_TRY(sh_launch_check(ctx, "cg_result"));
-        float lam = 1.0f;
-        for (int k = 0; k < 8; k++) {
-            SH_TRY(pwd_launch<NW>(ctx, 2, g, axis, x, W.p[cur], W.dp, lam, W.p[1 - cur], W, mask));
-            SH_TRY(finalize(ctx, W, nb_pw, 1, F_LS, it, n, k));
-            lam *= 0.5f;
-        }
+        SH_TRY(pwd_launch<NW>(ctx, 2, g, axis, x, W.p[cur], W.dp, 1.0f, W.p[1 - cur], W, mask));
+        SH_TRY(finalize(ctx, W, nb_pw, 1, F_LS0, it, n));
+        const float pmax = 3.402823466e+38f, pmin = -3.402823466e+38f;
+        const FastDiv f1((unsigned)g.n1), f2((unsigned)g.n2);
+        hipLaunchKernelGGL((pwd_halved<NW>), dim3(nb_pw), dim3(256), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax, g.n1,
+                           g.n2, g.n3, axis, W.part, W.sc, f1, f2);
+        SH_TRY(sh_launch_check(ctx, "pwd_halved"));
+        SH_TRY(finalize(ctx, W, nb_pw, LS_SUMS, F_LS7, it, n));
+        hipLaunchKernelGGL((pwd_chosen<NW>), dim3(nb_pw), dim3(256), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax,
+                           W.p[1 - cur], W.u2, g.n1, g.n2, g.n3, axis, W.sc, f1, f2);
+        SH_TRY(sh_launch_check(ctx, "pwd_chosen"));
         cur = 1 - cur;
     }
     *final_idx = cur;
@@ -975,7 +1053,8 @@ extern "C" int shd_dip(sh_ctx *ctx, const float *data, const float *mask, const 
     nblk_max = std::max<long>(nblk_max, (long)ceil_div(n1, F_TI1) * ceil_div(n2, F_TI2) * n3);
     nblk_max = std::max<long>(nblk_max, DIP_GRID_CAP);  // every capped launch, whatever its tile
     W.nblk_max = (int)nblk_max;
-    SH_TRY(sh_slot(ctx, SLOT_RED, (size_t)nblk_max * 3 * sizeof(double), (void **)&W.part));
+    const size_t npart = std::max<size_t>((size_t)nblk_max * 3, (size_t)DIP_GRID_CAP * LS_SUMS);
+    SH_TRY(sh_slot(ctx, SLOT_RED, npart * sizeof(double), (void **)&W.part));
     SH_TRY(sh_slot(ctx, SLOT_SCAL, sizeof(DipScal), (void **)&W.sc));
     SH_HIP(ctx, hipMemsetAsync(W.sc, 0, sizeof(DipScal), ctx->stream));
     if (mask) {
@@ -1005,7 +1084,7 @@ extern "C" int shd_dip(sh_ctx *ctx, const float *data, const float *mask, const 
                               &W2.sp, &W2.sx, &W2.sr, &W2.gp, &W2.pc, &W2.t1, &W2.t2, &W2.dp};
         for (int q = 0; q < NF; q++) *slots2[q] = fbuf2 + (size_t)q * n;
         W2.nblk_max = W.nblk_max;
-        SH_TRY(sh_slot(ctx, SLOT_DIP0 + 3, (size_t)nblk_max * 3 * sizeof(double), (void **)&W2.part));
+        SH_TRY(sh_slot(ctx, SLOT_DIP0 + 3, npart * sizeof(double), (void **)&W2.part));
         SH_TRY(sh_slot(ctx, SLOT_DIP0 + 4, sizeof(DipScal), (void **)&W2.sc));
         SH_HIP(ctx, hipMemsetAsync(W2.sc, 0, sizeof(DipScal), ctx->stream));
         SH_HIP(ctx, hipEventRecord(ctx->ev_fork, ctx->stream));

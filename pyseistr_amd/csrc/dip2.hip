@@ -198,7 +198,7 @@ d2_resident(const Resident R) {
     // one barrier with sums, then the scalar step
     auto step = [&](auto &v, int mode, int it) {
         fine = meet(R, ++epoch, v, sh, tot, &ok);
-        if (tid == 0 && fine) dip_scalar_step(&s, tot, mode, it, n, 1.e-6f, 0);
+        if (tid == 0 && fine) dip_scalar_step(&s, tot, mode, it, n, 1.e-6f);
         __syncthreads();
     };
     {
@@ -285,8 +285,8 @@ d2_resident(const Resident R) {
                 }
             fine = meet(R, ++epoch, v, sh, tot, &ok);
             if (tid == 0 && fine) {
-                if (k == 0) dip_scalar_step(&s, tot + 1, F_R0, it, n, 1.e-6f, 0);  // zero residual: zero model
-                dip_scalar_step(&s, tot, F_GN, k, n, 1.e-6f, 0);
+                if (k == 0) dip_scalar_step(&s, tot + 1, F_R0, it, n, 1.e-6f);  // zero residual: zero model
+                dip_scalar_step(&s, tot, F_GN, k, n, 1.e-6f);
             }
             __syncthreads();
             if (!fine || s.cg_done) break;

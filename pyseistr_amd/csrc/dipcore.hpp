@@ -31,7 +31,7 @@ struct DipScal {
     int rec[2 * 64];    // per GN iteration (first 64): cg iterations, accepted step
 };
 
-enum { F_USUM = 0, F_DIVN, F_R0, F_GN, F_BETA, F_LS, F_LS0, F_LS7 };
+enum { F_USUM = 0, F_DIVN, F_R0, F_GN, F_BETA, F_LS0, F_LS7 };
 
 // fold position q (may lie outside [0,n)) back by even reflection
 __device__ inline int fold_idx(int q, int n) {
@@ -43,8 +43,7 @@ __device__ inline int fold_idx(int q, int n) {
 
 // Scalar logic of one finalize step of a dip direction, given the reduced
 // sums tot[] of the preceding kernel (thread 0 only).
-__device__ inline void dip_scalar_step(DipScal *sc, const double *tot, int mode, int it, long n, float tol,
-                                       int k_ls) {
+__device__ inline void dip_scalar_step(DipScal *sc, const double *tot, int mode, int it, long n, float tol) {
     switch (mode) {
     case F_USUM:
         sc->usum = tot[0];
@@ -93,19 +92,7 @@ __device__ inline void dip_scalar_step(DipScal *sc, const double *tot, int mode,
             sc->cg_iters = it + 1;
         }
         break;
-    case F_LS:  // dip_cfuns.c:1667-1687: accept on strict decrease
-        if (sc->accepted) break;
-        if (tot[0] < sc->usum || k_ls == 7) {
-            sc->accepted = (tot[0] < sc->usum) ? 1 : 2;
-            sc->ls_k = (tot[0] < sc->usum) ? k_ls : 8;
-            sc->usum = tot[0];
-            if (it < 64) {
-                sc->rec[2 * it] = sc->cg_iters;
-                sc->rec[2 * it + 1] = sc->ls_k;
-            }
-        }
-        break;
-    case F_LS0:  // the full step alone
+    case F_LS0:  // the full step (dip_cfuns.c:1667-1687: accept on strict decrease)
         if (tot[0] < sc->usum) {
             sc->accepted = 1;
             sc->ls_k = 0;
