@@ -184,6 +184,108 @@ cg_result_kernel(const float *__restrict__ xa, const float *__restrict__ xb, con
 
 
 
+// Axes 1 and 2 in one pass, over tiles of a plane (i3) with halos; the field
+// between the two stays in LDS.  The folded columns and rows of a tile are
+// tabled once, so a staged sample costs two table reads and its loads, BL of
+// which a thread has in flight; the stencils give four outputs a read pair
+// (their operations are those of the passes below, in the same order).  A
+// block runs a contiguous range of tiles, the XCDs contiguous runs of blocks.
+// Four fields less an iteration of the CG than one axis a pass.  A dip of 256
+// x 128 x 128, rect 5: 10.1 -> 8.5 ms (rect 20, halos as large as the tile:
+// 10.0 -> 9.4); 512 x 256 x 256: 22.5 -> 21.9 ms; 250 x 100 x 50: 5.9 -> 4.5.
+// Tiles of 64 x 16: 8.7 (512 x 256 x 256: 22.4), of 32 x 8: 11.1 ms.
+constexpr int P12_T1 = 64, P12_T2 = 32;
+inline SH_HD int p12_row(int nb1) { return P12_T1 + 2 * (nb1 - 1) + 1; }  // odd: rows start at different banks
+inline size_t p12_lds(int nb1, int nb2) {
+    const size_t R2 = P12_T2 + 2 * ((size_t)nb2 - 1);
+    return sizeof(float) * (R2 * (p12_row(nb1) + P12_T1)) + sizeof(unsigned) * (p12_row(nb1) + R2);
+}
+
+template <int PRO, bool NT>
+__global__ void __launch_bounds__(256)
+smooth_pair12(const float *__restrict__ in, float *__restrict__ out, int n1, int n2, long ntask, int nb1, int nb2,
+              CgArgs A, const DipScal *sc) {
+    if (sc->cg_done) return;
+    constexpr int T1 = P12_T1, T2 = P12_T2;
+    extern __shared__ float lds[];
+    __shared__ float w1[SM_HMAX + 1], w2[SM_HMAX + 1];
+    const int h1 = nb1 - 1, h2 = nb2 - 1, W1 = T1 + 2 * h1, WP = p12_row(nb1), R2 = T2 + 2 * h2, tid = threadIdx.x;
+    float *tile = lds, *s1 = tile + R2 * WP;  // [R2][WP], [R2][T1]
+    unsigned *cx = (unsigned *)(s1 + R2 * T1), *cy = cx + WP;
+    const bool pend = PRO == PRO_CG && sc->pending != 0;
+    const float a2 = pend ? (float)sc->alpha2 : 0.0f;
+    const int cur = (PRO == PRO_CG) ? sc->cur : 0;
+    sm_weights(w1, nb1);
+    sm_weights(w2, nb2);
+    const int nt1 = (n1 + T1 - 1) / T1, nt2 = (n2 + T2 - 1) / T2;
+    const long run = (long)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;  // gridDim.x: a multiple of 8
+    const long per = (ntask + gridDim.x - 1) / gridDim.x, t0 = run * per, t1 = min(ntask, t0 + per);
+    const int dr = 256 / W1, dc = 256 - dr * W1, r0 = tid / W1, c0 = tid - r0 * W1;
+    for (long task = t0; task < t1; task++) {
+        const int x0 = (int)(task % nt1) * T1, y0 = (int)(task / nt1 % nt2) * T2;
+        const long off = task / ((long)nt1 * nt2) * n1 * n2;  // the plane
+        __syncthreads();  // the last tile's readers are done with cx, cy and s1
+        for (int k = tid; k < W1; k += 256) cx[k] = fold_idx(x0 - h1 + k, n1);
+        for (int k = tid; k < R2; k += 256) cy[k] = (unsigned)fold_idx(y0 - h2 + k, n2) * (unsigned)n1;
+        auto at = [&](auto *p) { return p + off; };
+        const CgArgs B = PRO == PRO_CG ? CgArgs{at(A.w), at(A.xa), at(A.xb), at(A.ra), at(A.rb), at(A.sx), at(A.sr),
+                                                nullptr, nullptr, nullptr}
+                                       : CgArgs{};
+        const float *src = PRO == PRO_PLAIN ? in + off : nullptr;
+        const int oc = min(T1, n1 - x0), orow = min(T2, n2 - y0);  // own columns and rows
+        __syncthreads();
+        constexpr int BL = PRO == PRO_CG ? 4 : 8;
+        int r = r0, c = c0;
+        for (int e0 = tid; e0 < R2 * W1; e0 += BL * 256) {
+            float raw[BL][5];
+            int rr[BL], cc[BL];
+            unsigned gi[BL];
+#pragma unroll
+            for (int b = 0; b < BL; b++) {
+                rr[b] = min(r, R2 - 1);
+                cc[b] = c;
+                gi[b] = cx[c] + cy[rr[b]];
+                sm_fetch<PRO>(src, gi[b], B, pend, cur, raw[b]);
+                if (r >= R2) rr[b] = -1;
+                r += dr;
+                c += dc;
+                if (c >= W1) {
+                    c -= W1;
+                    r++;
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < BL; b++)
+                if (rr[b] >= 0) {
+                    const bool own = (unsigned)(cc[b] - h1) < (unsigned)oc && (unsigned)(rr[b] - h2) < (unsigned)orow;
+                    tile[rr[b] * WP + cc[b]] = sm_finish<PRO>(raw[b], gi[b], own, B, pend, a2, cur);
+                }
+        }
+        __syncthreads();
+        for (int e = tid; e < R2 * (T1 / 4); e += 256) {
+            const int q = e / (T1 / 4), k = e % (T1 / 4) * 4;
+            float o[4];
+            tri4(tile + q * WP + k + h1, 1, w1, h1, o);
+#pragma unroll
+            for (int j = 0; j < 4; j++) s1[q * T1 + k + j] = o[j];
+        }
+        __syncthreads();
+        for (int e = tid; e < T2 / 4 * T1; e += 256) {
+            const int q = e / T1 * 4, k = e % T1;
+            float o[4];
+            tri4(s1 + (q + h2) * T1 + k, T1, w2, h2, o);
+            if (k < oc)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (q + j < orow) {
+                        float *p = out + off + (unsigned)(x0 + k) + (unsigned)n1 * (unsigned)(y0 + q + j);
+                        if (NT) st_nt(p, o[j]);
+                        else *p = o[j];
+                    }
+        }
+    }
+}
+
 // Axis 1 (contiguous): task = one chunk of one trace; a block runs a
 // contiguous range of tasks (ntask = chunks * traces).
 template <int PRO, int EPI, bool NT = false>
@@ -671,6 +773,7 @@ struct SmoothPlan {
     int naxes;
     int axis[3];
     int nb[3];
+    bool pair12;  // axes 1 and 2 in one pass (smooth_pair12), axis 3 after it
     int fused;  // all axes in one pass (smooth_fused)
     int r[3];   // radius per axis (1 = inactive)
 };
@@ -773,7 +876,25 @@ int smooth_apply(sh_ctx *ctx, const DipGeom &g, const SmoothPlan &sp, const floa
     // with non-temporal stores (their arrays do not stay in the L2)
     const bool nt = g.n >= (1L << 24);
     const float *src = in;
-    for (int a = 0; a < nsep; a++) {
+    int a0 = 0;
+    if (sp.pair12) {
+        const long ntask = (long)ceil_div(g.n1, P12_T1) * ceil_div(g.n2, P12_T2) * g.n3;
+        const dim3 grid((unsigned)std::min<long>(ceil_div(ntask, 8) * 8L, DIP_GRID_CAP));
+        const size_t lds = p12_lds(sp.nb[0], sp.nb[1]);
+        PROF_A(ctx);
+#define SM_P12(PP, NN)                                                                                             \
+    hipLaunchKernelGGL((smooth_pair12<PP, NN>), grid, dim3(256), lds, ctx->stream, src, W.t1, g.n1, g.n2, ntask,   \
+                       sp.nb[0], sp.nb[1], A, W.sc)
+        if (pro == PRO_CG) { if (nt) SM_P12(PRO_CG, true); else SM_P12(PRO_CG, false); }
+        else { if (nt) SM_P12(PRO_PLAIN, true); else SM_P12(PRO_PLAIN, false); }
+#undef SM_P12
+        PROF_B(ctx, pro == PRO_CG ? "smooth_pair12<1>" : "smooth_pair12<0>",
+               pass_bytes(pro, EPI_PLAIN, first != 0, false) * (double)g.n);
+        SH_TRY(sh_launch_check(ctx, "smooth_pair12"));
+        src = W.t1;
+        a0 = 2;
+    }
+    for (int a = a0; a < nsep; a++) {
         bool is_first = a == 0, is_last = a == sp.naxes - 1;
         int P = is_first ? pro : PRO_PLAIN;
         int E = is_last ? epi : EPI_PLAIN;
@@ -1003,6 +1124,11 @@ extern "C" int shd_dip(sh_ctx *ctx, const float *data, const float *mask, const 
         if (env && env[0] == '3' && plan.naxes == 3 && plan.r[1] - 1 <= P_HMAX2 && plan.r[2] >= 2 && plan.r[2] <= 7)
             plan.fused = 3;
     }
+    // axes 1 and 2 in one pass where both are smoothed before the last one and
+    // the tile fits (faster at every size and radius measured, up to the
+    // largest that fits).  The switches of the separable passes select those.
+    plan.pair12 = plan.naxes == 3 && !plan.fused && !getenv("SH_SMOOTH_TILE") && !getenv("SH_SMOOTH_WAVE") &&
+                  !getenv("SH_SMOOTH_COL") && p12_lds(plan.nb[0], plan.nb[1]) <= 60 * 1024;
     // a 2-D section that fits the chip: resident, in one launch (dip2.hip).
     // The switches of the smoothing passes select the launches.
     if (n3 == 1 && r3 <= 1 && !getenv("SH_SMOOTH_FUSED") && !getenv("SH_SMOOTH_TILE") && !getenv("SH_SMOOTH_WAVE") &&
