@@ -246,6 +246,45 @@ __device__ inline void fac_row(const BFactor &F, long k, float *ok) {
     }
 }
 
+// One node's prediction at target trace j through buffer resources; tid: the
+// thread's column of the launch's scratch (cnt * gx8 * TB of them).
+template <int NW, int NF, int PF>
+__device__ inline void level_node(const float *pi, const float *px, float *U, const float *F, const Node3 &nd, int cnt,
+                                  long gx8, long j, long tid, int n1, int n2, long ntr, int np2, float e, float *scr) {
+    constexpr int NB = 2 * NW;
+    const long n = (long)n1 * ntr;
+    // NF == 2: axis 2 then axis 3; NF == 1: the node's one axis
+    const unsigned row = (unsigned)ntr * 4u;
+    BTrace in[2], q[2];
+    bool rev[2];
+    const bool ax2 = (nd.update & 1) != 0;
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        const bool a2 = NF == 2 ? f == 0 : ax2;
+        const int up = a2 ? nd.up2 : nd.up3;
+        const long d = a2 ? 1 : n2;
+        const int ks = nd.slot + (up ? -1 : 1) * (a2 ? 1 : np2);
+        in[f] = BTrace{plane_rsrc(U + (long)ks * n, (unsigned long)n * 4), (unsigned)(up ? j - d : j + d) * 4u,
+                       row};
+        q[f] = BTrace{plane_rsrc(a2 ? pi : px, (unsigned long)n * 4), (unsigned)(up ? j - d : j) * 4u, row};
+        rev[f] = up != 0;
+    }
+    const float *Fp = F + (long)node_variant(nd.update, nd.up2, nd.up3) * fac_plane_floats(NB, n);
+    const BFactor Fv{plane_rsrc(Fp + (long)NB * n, (unsigned long)n * 4),
+                     plane_rsrc(Fp, (unsigned long)n * NB * 4),
+                     (unsigned)j * 4u,
+                     (unsigned)j * (4u * NB),
+                     row,
+                     row * NB};
+    const unsigned lt = (unsigned)(cnt * gx8 * TB);  // threads of this launch
+    // scratch written and read with non-temporal accesses (keeps the
+    // shared factor and slope lines in the L2)
+    const BSinkNT y{plane_rsrc(scr, (unsigned long)lt * n1 * 4), (unsigned)tid * 4u, lt * 4u};
+    // the slot is read only by later levels and the median: non-temporal
+    const BSinkNT o{plane_rsrc(U + (long)nd.slot * n, (unsigned long)n * 4), (unsigned)j * 4u, row};
+    solve_factored_pf<NW, NF, PF>(in, q, rev, Fv, y, n1, e, o);
+}
+
 // One launch per (level, number of source traces NF): every thread predicts
 // one slot at one target trace with the shared factor of the target.  A
 // slot whose source lies outside the volume is written as zeros there
@@ -277,36 +316,7 @@ spray3_level(const float *__restrict__ pi, const float *__restrict__ px, float *
     long tid = (long)node * gx8 * TB + j;
     constexpr int NB = 2 * NW;
     if constexpr (BUF && PF > 0) {
-        // NF == 2: axis 2 then axis 3; NF == 1: the node's one axis
-        const unsigned row = (unsigned)ntr * 4u;
-        BTrace in[2], q[2];
-        bool rev[2];
-        const bool ax2 = (nd.update & 1) != 0;
-#pragma unroll
-        for (int f = 0; f < NF; f++) {
-            const bool a2 = NF == 2 ? f == 0 : ax2;
-            const int up = a2 ? nd.up2 : nd.up3;
-            const long d = a2 ? 1 : n2;
-            const int ks = nd.slot + (up ? -1 : 1) * (a2 ? 1 : np2);
-            in[f] = BTrace{plane_rsrc(U + (long)ks * n, (unsigned long)n * 4), (unsigned)(up ? j - d : j + d) * 4u,
-                           row};
-            q[f] = BTrace{plane_rsrc(a2 ? pi : px, (unsigned long)n * 4), (unsigned)(up ? j - d : j) * 4u, row};
-            rev[f] = up != 0;
-        }
-        const float *Fp = F + (long)node_variant(nd.update, nd.up2, nd.up3) * fac_plane_floats(NB, n);
-        const BFactor Fv{plane_rsrc(Fp + (long)NB * n, (unsigned long)n * 4),
-                         plane_rsrc(Fp, (unsigned long)n * NB * 4),
-                         (unsigned)j * 4u,
-                         (unsigned)j * (4u * NB),
-                         row,
-                         row * NB};
-        const unsigned lt = (unsigned)(cnt * gx8 * TB);  // threads of this launch
-        // scratch written and read with non-temporal accesses (keeps the
-        // shared factor and slope lines in the L2)
-        const BSinkNT y{plane_rsrc(scr, (unsigned long)lt * n1 * 4), (unsigned)tid * 4u, lt * 4u};
-        // the slot is read only by later levels and the median: non-temporal
-        const BSinkNT o{plane_rsrc(U + (long)nd.slot * n, (unsigned long)n * 4), (unsigned)j * 4u, row};
-        solve_factored_pf<NW, NF, PF>(in, q, rev, Fv, y, n1, e, o);
+        level_node<NW, NF, PF>(pi, px, U, F, nd, cnt, gx8, j, tid, n1, n2, ntr, np2, e, scr);
         return;
     }
     Sink y{scr + tid, nthr};
@@ -335,6 +345,30 @@ spray3_level(const float *__restrict__ pi, const float *__restrict__ px, float *
         solve_factored_pf<NW, NF, PF>(in, q, rev, Fv, y, n1, e, out);
     else
         solve_factored<NW, NF>(in, q, rev, Fv, y, n1, e, out);
+}
+
+// A level's one- and two-source nodes in one launch (they are independent of
+// each other), each as spray3_level runs it.
+template <int NW>
+__global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(NW <= 2 ? 2 : 1)))
+spray3_both(const float *__restrict__ pi, const float *__restrict__ px, float *__restrict__ U,
+            const float *__restrict__ F, const Level3 nodes, int cnt, int xcd, int n1, int n2, int n3, int np2,
+            float e, float *__restrict__ scr) {
+    const long ntr = (long)n2 * n3, n = (long)n1 * ntr, gx8 = (ntr + 8L * TB - 1) / (8L * TB) * 8;
+    long jb;
+    const int node = level_block(xcd, cnt, gx8, jb);
+    const long j = jb * TB + threadIdx.x;
+    if (j >= ntr) return;
+    const Node3 nd = nodes.nd[node];
+    const int i2 = (int)(j % n2) - nd.o2, i3 = (int)(j / n2) - nd.o3;
+    if (i2 < 0 || i2 >= n2 || i3 < 0 || i3 >= n3) {
+        float *out = U + (long)nd.slot * n + j;
+        for (int k = 0; k < n1; k++) out[k * ntr] = 0.0f;
+        return;
+    }
+    const long tid = (long)node * gx8 * TB + j;
+    if (nd.update == 3) level_node<NW, 2, 6>(pi, px, U, F, nd, cnt, gx8, j, tid, n1, n2, ntr, np2, e, scr);
+    else level_node<NW, 1, 8>(pi, px, U, F, nd, cnt, gx8, j, tid, n1, n2, ntr, np2, e, scr);
 }
 
 // Two-source slots grouped by (level, quadrant): every slot of a group
@@ -814,6 +848,27 @@ int spray3_run(sh_ctx *ctx, int order, int n1, int n2, int n3, int ns2, int ns3,
                 PROF_B(ctx, "spray3_group", by);
                 SH_TRY(sh_launch_check(ctx, "spray3_group"));
             }
+        }
+        // both kinds in one launch where one alone leaves the chip's two
+        // waves a SIMD (512 blocks) idle: up to twice that many blocks
+        // together.  somf3d, r = 4: 251 x 60 x 60 2.00 -> 1.56 ms, 251 x 127
+        // x 121 2.08 -> 1.91, 300 x 256 x 256 8.26 -> 8.16 (beyond the line).
+        const long all = (long)levels[L].size(), two = std::count_if(levels[L].begin(), levels[L].end(),
+                                                                     [](const Node3 &nd) { return nd.update == 3; });
+        if (!grouped && !pe && !(be && be[0] == '0') && two && two < all && gx8 * all <= 1024 &&
+            (double)n * 4 * (2 * order) < 4294967296.0 && (double)gx8 * TB * all * n1 * 4 < 4294967296.0) {
+            Level3 lv{};
+            int cnt = 0;
+            for (int v = 0; v < 8; v++)
+                for (auto &nd : levels[L])
+                    if (node_variant(nd.update, nd.up2, nd.up3) == v) lv.nd[cnt++] = nd;
+            PROF_A(ctx);
+            SH_DISPATCH_NW(ctx, order, NW,
+                           hipLaunchKernelGGL((spray3_both<NW>), dim3((unsigned)(gx8 * cnt)), dim3(TB), 0, ctx->stream, piT,
+                                              pxT, U, F, lv, cnt, xcd, n1, n2, n3, np2, e, scr));
+            PROF_B(ctx, "spray3_both", (20.0 * two + 12.0 * (all - two)) * (double)n);
+            SH_TRY(sh_launch_check(ctx, "spray3_both"));
+            continue;
         }
         for (int nf = 1; nf <= (grouped ? 1 : 2); nf++) {
             Level3 lv{};

@@ -232,6 +232,21 @@ def test_pwd_ranges_equal_single_samples(ps, monkeypatch, shape, order, njs):
     assert np.abs(new - old).max() <= 5 * 8 * 2.0**-24 * max(np.abs(old).max(), 1.0)
 
 
+@pytest.mark.parametrize("shape,r,order", [((40, 9, 8), (1, 1), 1), ((33, 16, 16), (2, 3), 2), ((64, 17, 15), (3, 0), 2),
+                                           ((24, 64, 33), (4, 4), 2), ((9, 3, 2), (4, 4), 1), ((30, 50, 41), (2, 2), 3)])
+def test_levels_in_one_launch_equal_two(ps, monkeypatch, shape, r, order):
+    """A spray level's one- and two-source nodes in one launch and in one
+    each (SH_SPRAY_PF selects the latter): the same bits, from volumes
+    smaller than the radius to a few blocks of traces."""
+    d, _, p, q = _case3(shape, 5)
+    kw = dict(order=order, eps=0.01, verb=0)
+    new = [ps.somf3dc(d, p, q, r[0], r[1], **kw), ps.somean3dc(d, p, q, r[0], r[1], **kw)]
+    monkeypatch.setenv("SH_SPRAY_PF", "6")
+    old = [ps.somf3dc(d, p, q, r[0], r[1], **kw), ps.somean3dc(d, p, q, r[0], r[1], **kw)]
+    for a, b in zip(new, old):
+        same(a, b, str(shape))
+
+
 @pytest.mark.parametrize("shape,rect", [((64, 32, 5), (5, 5, 5)), ((65, 33, 4), (2, 9, 3)), ((63, 31, 6), (9, 2, 2)),
                                         ((129, 7, 8), (5, 12, 2)), ((9, 40, 7), (13, 3, 4)), ((3, 2, 2), (4, 5, 2)),
                                         ((200, 95, 3), (20, 27, 2)), ((70, 40, 500), (3, 3, 3)), ((130, 70, 3), (40, 2, 2))])
