@@ -83,10 +83,12 @@ __device__ inline void covering(int i, int l, int s, int P, int &lo, int &hi) {
 // One block per (i2, i3) column of the output, threads along i1.  Every
 // sample adds its covering patches in patch order (p1, then p2, then p3),
 // the order in which the reference accumulates them.  Bound by reading X,
-// each value once: the loads are non-temporal, of four samples at a time.
-// 6000 x 2500 in patches of 256 x 128, half overlapping (0.48 GB of patches):
-// 167 us with one load in flight, 137 with four, 115 non-temporal (the copy's
-// rate takes 128 us).
+// each value once, U samples of a thread at a time (as many as a
+// trace gives 256 threads, up to four).  6000 x 2500 in patches of 256 x 128,
+// half overlapping (0.48 GB of patches): 167 us with one load in flight, 137
+// with four, 115 non-temporal (the copy's rate takes 128 us); 512 x 256 x 256
+// in 64 x 32 x 32: 430 -> 358.
+template <int U, bool NT>
 __global__ void patch_paste(const double *__restrict__ X, double *__restrict__ out, PGeo g, long L) {
     const int c = blockIdx.x;
     const int i2 = c % g.n[1], i3 = c / g.n[1];
@@ -94,7 +96,6 @@ __global__ void patch_paste(const double *__restrict__ X, double *__restrict__ o
     covering(i2, g.l[1], g.s[1], g.P[1], lo2, hi2);
     covering(i3, g.l[2], g.s[2], g.P[2], lo3, hi3);
     const long l1 = g.l[0], l12 = (long)g.l[0] * g.l[1];
-    constexpr int U = 4;  // samples of a thread whose loads are in flight together
     for (long i0 = threadIdx.x; i0 < g.n[0]; i0 += U * blockDim.x) {
         int lo1[U], hi1[U], most = 0;
         double acc[U], cnt[U];
@@ -112,13 +113,14 @@ __global__ void patch_paste(const double *__restrict__ X, double *__restrict__ o
 #pragma unroll
                     for (int u = 0; u < U; u++) {
                         const int i1 = (int)min(i0 + u * (long)blockDim.x, g.n[0] - 1L), p1 = lo1[u] + k;
-                        const bool on = p1 <= hi1[u];
+                        const bool on = U == 1 || p1 <= hi1[u];
                         const long id = ((long)p1 * g.P[1] + p2) * g.P[2] + p3;
-                        v[u] = __builtin_nontemporal_load(X + (on ? id * L + (i1 - p1 * g.s[0]) + e23 : 0));
+                        const double *p = X + (on ? id * L + (i1 - p1 * g.s[0]) + e23 : 0);
+                        v[u] = NT ? __builtin_nontemporal_load(p) : *p;
                     }
 #pragma unroll
                     for (int u = 0; u < U; u++)
-                        if (lo1[u] + k <= hi1[u]) {
+                        if (U == 1 || lo1[u] + k <= hi1[u]) {
                             acc[u] += v[u];
                             cnt[u] += 1.0;
                         }
@@ -188,6 +190,14 @@ extern "C" int sh_patch_inv(sh_ctx *ctx, const double *X, double *out, int n1, i
     long np, L;
     SH_TRY(geometry(ctx, n1, n2, n3, l1, l2, l3, s1, s2, s3, g, np, L));
     const int tpb = (int)std::min<long>(256, ceil_div((long)n1, 64) * 64);
-    hipLaunchKernelGGL(patch_paste, dim3((unsigned)((long)n2 * n3)), dim3(tpb), 0, ctx->stream, X, out, g, L);
+    const dim3 grid((unsigned)((long)n2 * n3));
+    // non-temporal where the patches are more than the Infinity Cache holds
+    // (200 x 100 x 100 in half-overlapping cubes of 32: 41 us, plain loads 32)
+    const bool nt = (size_t)np * L * sizeof(double) > (256u << 20);
+#define PP_(U, N) hipLaunchKernelGGL((patch_paste<U, N>), grid, dim3(tpb), 0, ctx->stream, X, out, g, L)
+    if (n1 > 3 * 256) { if (nt) PP_(4, true); else PP_(4, false); }
+    else if (n1 > 384) { if (nt) PP_(2, true); else PP_(2, false); }
+    else { if (nt) PP_(1, true); else PP_(1, false); }
+#undef PP_
     return sh_launch_check(ctx, "patch_paste");
 }
