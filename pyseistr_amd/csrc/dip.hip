@@ -189,10 +189,12 @@ cg_result_kernel(const float *__restrict__ xa, const float *__restrict__ xb, con
 // tabled once, so a staged sample costs two table reads and its loads, BL of
 // which a thread has in flight; the stencils give four outputs a read pair
 // (their operations are those of the passes below, in the same order).  A
-// block runs a contiguous range of tiles, the XCDs contiguous runs of blocks.
+// block runs a contiguous range of tiles, down axis 2 first (their halos, the
+// larger ones, are in the caches then: 512 x 256 x 256 21.7 -> 21.2 ms), the
+// XCDs contiguous runs of blocks.
 // Four fields less an iteration of the CG than one axis a pass.  A dip of 256
 // x 128 x 128, rect 5: 10.1 -> 8.5 ms (rect 20, halos as large as the tile:
-// 10.0 -> 9.4); 512 x 256 x 256: 22.5 -> 21.9 ms; 250 x 100 x 50: 5.9 -> 4.5.
+// 10.0 -> 9.4); 512 x 256 x 256: 22.5 -> 21.2 ms; 250 x 100 x 50: 5.9 -> 4.5.
 // Tiles of 64 x 16: 8.7 (512 x 256 x 256: 22.4), of 32 x 8: 11.1 ms.
 constexpr int P12_T1 = 64, P12_T2 = 32;
 inline SH_HD int p12_row(int nb1) { return P12_T1 + 2 * (nb1 - 1) + 1; }  // odd: rows start at different banks
@@ -222,7 +224,7 @@ smooth_pair12(const float *__restrict__ in, float *__restrict__ out, int n1, int
     const long per = (ntask + gridDim.x - 1) / gridDim.x, t0 = run * per, t1 = min(ntask, t0 + per);
     const int dr = 256 / W1, dc = 256 - dr * W1, r0 = tid / W1, c0 = tid - r0 * W1;
     for (long task = t0; task < t1; task++) {
-        const int x0 = (int)(task % nt1) * T1, y0 = (int)(task / nt1 % nt2) * T2;
+        const int y0 = (int)(task % nt2) * T2, x0 = (int)(task / nt2 % nt1) * T1;
         const long off = task / ((long)nt1 * nt2) * n1 * n2;  // the plane
         __syncthreads();  // the last tile's readers are done with cx, cy and s1
         for (int k = tid; k < W1; k += 256) cx[k] = fold_idx(x0 - h1 + k, n1);
