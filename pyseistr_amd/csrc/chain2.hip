@@ -80,14 +80,17 @@ __device__ inline __amdgpu_buffer_rsrc_t chain_rsrc(const void *p, unsigned long
 }
 
 // Row k of a plane of factor rows through a buffer resource: the lane's
-// offset in a register, the row's as the instruction's scalar offset.
+// offset in a register, the row's as the instruction's scalar offset, which
+// the resource's range check does not cover: rows past the last one are read
+// as the last one.
 template <int NB>
 struct ChainRows {
     __amdgpu_buffer_rsrc_t r;
     int lane;      // byte offset of the trace's row 0
     unsigned row;  // bytes from one sample to the next
+    int last;      // the last row
     __device__ void load(int k, float *o) const {
-        const int so = (int)__builtin_amdgcn_readfirstlane((unsigned)k * row);
+        const int so = (int)__builtin_amdgcn_readfirstlane((unsigned)min(k, last) * row);
         typedef float f2 __attribute__((ext_vector_type(2)));
         if constexpr (NB % 4 == 0) {
 #pragma unroll
@@ -111,8 +114,7 @@ struct ChainRows {
 // Forward substitution in place over the LDS row y (banded_solve's first
 // loop): y[k] -= o_m[k-1-m] y[k-1-m], m = 0 .. NB-1 in turn.  Entries before
 // the trace are zeros (subtracting 0 * 0 changes nothing); the last group
-// runs on into the row's padding, which nothing reads.  Factor rows past the
-// slice read as zeros.
+// runs on into the row's padding, which nothing reads.
 template <int NB, int D>
 __device__ inline void chain_forward(const ChainRows<NB> &F, float *y, int n1) {
     float o[D][NB], b[NB];
@@ -155,13 +157,17 @@ __device__ inline void chain_forward(const ChainRows<NB> &F, float *y, int n1) {
 
 // Backward substitution in place (banded_solve's second loop after the
 // division): y[k] -= o_m[k] y[k+1+m], from the end of the padding (zeros
-// there, and zero factor rows: its values stay zero).
+// there, and its factor rows are taken as zeros: its values stay zero).
 template <int NB, int D>
 __device__ inline void chain_backward(const ChainRows<NB> &F, float *y, int n1) {
     const int top = (n1 + D - 1) / D * D;
     float o[D][NB], x[NB];
 #pragma unroll
-    for (int s = 0; s < D; s++) F.load(top - D + s, o[s]);
+    for (int s = 0; s < D; s++) {
+        F.load(top - D + s, o[s]);
+#pragma unroll
+        for (int m = 0; m < NB; m++) o[s][m] = top - D + s < n1 ? o[s][m] : 0.0f;
+    }
 #pragma unroll
     for (int m = 0; m < NB; m++) x[m] = 0.0f;
     constexpr int R = 2;
@@ -298,7 +304,8 @@ __device__ inline void chain_solve(const ChainBlock &B, float *row, const float 
     // diagonal plane behind those of all slices
     const float *fo = Fv + (long)NB * B.base, *fd = Fv + (long)NB * n + B.base;
     const bool walker = threadIdx.x < (unsigned)B.nt && act;
-    const ChainRows<NB> F{chain_rsrc(fo, (unsigned long)B.slice * NB * 4), ip * NB * 4, (unsigned)B.n2 * NB * 4};
+    const ChainRows<NB> F{chain_rsrc(fo, (unsigned long)B.slice * NB * 4), ip * NB * 4, (unsigned)B.n2 * NB * 4,
+                          B.n1 - 1};
     __syncthreads();
     if (walker) {
         __builtin_amdgcn_s_setprio(3);

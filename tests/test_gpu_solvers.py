@@ -159,6 +159,37 @@ def test_chain_blocks_equal_single_threads(ps, monkeypatch, n1, n2, n3, ns, orde
         same(x, y, f"call {k}")
 
 
+@pytest.mark.parametrize("n1,n2,order", [(8, 1, 1), (9, 3, 2), (30, 40, 3), (21, 17, 4), (33, 70, 2), (65, 8, 2), (515, 9, 2)])
+def test_chain_blocks_take_nothing_past_the_factors(ps, monkeypatch, n1, n2, order):
+    """The block chains read whole groups of factor rows, past a trace's last
+    one where its length is no multiple: with NaN all over the workspace
+    before every call, the same bits as one thread per chain."""
+    from pyseistr_amd import filters
+    rng = np.random.default_rng(n1)
+    d = rng.standard_normal((n1, n2)).astype(np.float32)
+    p = rng.uniform(-2, 2, (n1, n2)).astype(np.float32)
+    u = rng.standard_normal(n1 * n2 * 5).astype(np.float32)
+    big = np.ones((600, 96), np.float32)
+
+    def dirty():
+        monkeypatch.setenv("SH_SPRAY2_PF", "8")  # writes every plane of the factors' buffer
+        filters.pwspray2d(big, np.nan * big, 1, 4, 0.01)
+        ps.somean2dc(big, np.nan * big, 1, 4, 0.01)
+        monkeypatch.delenv("SH_SPRAY2_PF")
+
+    calls = [lambda: filters.pwspray2d(d, p, 2, order, 0.01),
+             lambda: filters.pwspray2d_adjoint(u, p, 2, order, 0.01, (n1, n2)),
+             lambda: ps.somean2dc(d, p, 2, order, 0.01), lambda: ps.somean2dc(d, p, 2, order, 0.01, adj=1)]
+    for k, f in enumerate(calls):
+        dirty()
+        a = f()
+        monkeypatch.setenv("SH_SPRAY2_PF", "8")
+        b = f()
+        monkeypatch.delenv("SH_SPRAY2_PF")
+        assert np.isfinite(a).all()
+        same(a, b, f"call {k}")
+
+
 def test_spray3_level_paths_identical(ps, monkeypatch):
     """The 3-D spray levels give the same bits through buffer resources (the
     default) and through pointers (SH_SPRAY_BUF=0), at every prefetch
