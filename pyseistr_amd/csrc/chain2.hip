@@ -538,8 +538,10 @@ chain2_ldl(float *__restrict__ F, int n1, int n2, int n3) {
 }  // namespace
 
 bool chain2_fits(int n1, int n2, int n3, int order) {
-    // (a slice's factor rows are addressed with 32-bit offsets)
-    return n3 <= 65535 && (double)n1 * n2 * 8 * order < 4294967295.0 && chain_plan(n1, n2, n3, order).nt > 0;
+    // (a slice's factor rows are addressed with 32-bit offsets; the forward
+    // smoothing sprays two inputs at once, which is planned as 2 n3 slices)
+    return n3 <= 65535 && (double)n1 * n2 * 8 * order < 4294967295.0 && chain_plan(n1, n2, n3, order).nt > 0 &&
+           chain_plan(n1, n2, 2L * n3, order).nt > 0;
 }
 
 int chain2_factor(sh_ctx *ctx, const Pwsmooth2 &P) {
@@ -570,6 +572,7 @@ int chain2_factor(sh_ctx *ctx, const Pwsmooth2 &P) {
 int chain2_forward(sh_ctx *ctx, const Pwsmooth2 &P, const float *x, const float *x2, float *U2) {
     const int sprays = x2 ? 2 : 1;
     const ChainPlan K = chain_plan(P.n1, P.n2, (long)P.n3 * sprays, P.order);
+    if (K.nt < 1) return sh_fail(ctx, SH_EUNSUP, "chain2: traces of %d samples do not fit", P.n1);
     const dim3 grid(2 * K.nb, P.n3, sprays);
     CHAIN_DISPATCH(ctx, P.order, K.D,
                    hipLaunchKernelGGL((chain2_fwd<NW, DD>), grid, dim3(K.tb), K.lds, ctx->stream, x, P.dip, P.F, P.U, P.n1,
@@ -579,6 +582,7 @@ int chain2_forward(sh_ctx *ctx, const Pwsmooth2 &P, const float *x, const float 
 
 int chain2_adjoint(sh_ctx *ctx, const Pwsmooth2 &P, const float *U, const float *ww) {
     const ChainPlan K = chain_plan(P.n1, P.n2, P.n3, P.order);
+    if (K.nt < 1) return sh_fail(ctx, SH_EUNSUP, "chain2: traces of %d samples do not fit", P.n1);
     const dim3 grid(2 * K.nb, P.n3);
     CHAIN_DISPATCH(ctx, P.order, K.D,
                    hipLaunchKernelGGL((chain2_adj<NW, DD>), grid, dim3(K.tb), K.lds, ctx->stream, U, ww, P.dip, P.F, P.C,

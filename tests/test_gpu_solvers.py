@@ -190,6 +190,25 @@ def test_chain_blocks_take_nothing_past_the_factors(ps, monkeypatch, n1, n2, ord
         same(a, b, f"call {k}")
 
 
+@pytest.mark.parametrize("n1,n2,order", [(15000, 600, 2), (15150, 513, 1), (14600, 1024, 3), (14400, 700, 4), (15000, 3, 2),
+                                         (15352, 2, 1), (16000, 2, 1), (130, 1100, 2), (300, 1100, 1)])
+def test_chain_block_limits(ps, monkeypatch, n1, n2, order):
+    """The longest traces that blocks of chains hold, with one spray and with
+    two at once (the forward smoothing), and past them, where each chain has
+    a thread; more than 2048 chains with several pieces a trace: the same
+    bits as one thread per chain."""
+    from pyseistr_amd import filters
+    rng = np.random.default_rng(n1)
+    d = rng.standard_normal((n1, n2)).astype(np.float32)
+    p = rng.uniform(-2, 2, (n1, n2)).astype(np.float32)
+    calls = [lambda: filters.pwspray2d(d, p, 1, order, 0.01), lambda: ps.somean2dc(d, p, 1, order, 0.01),
+             lambda: ps.somean2dc(d, p, 1, order, 0.01, adj=1)]
+    a = [f() for f in calls]
+    monkeypatch.setenv("SH_SPRAY2_PF", "8")
+    for k, f in enumerate(calls):
+        same(a[k], f(), f"call {k}")
+
+
 def test_spray3_level_paths_identical(ps, monkeypatch):
     """The 3-D spray levels give the same bits through buffer resources (the
     default) and through pointers (SH_SPRAY_BUF=0), at every prefetch
