@@ -537,11 +537,23 @@ chain2_ldl(float *__restrict__ F, int n1, int n2, int n3) {
 
 }  // namespace
 
-bool chain2_fits(int n1, int n2, int n3, int order) {
-    // (a slice's factor rows are addressed with 32-bit offsets; the forward
-    // smoothing sprays two inputs at once, which is planned as 2 n3 slices)
-    return n3 <= 65535 && (double)n1 * n2 * 8 * order < 4294967295.0 && chain_plan(n1, n2, n3, order).nt > 0 &&
-           chain_plan(n1, n2, 2L * n3, order).nt > 0;
+// Whether the blocks run (one thread per chain otherwise).  A block's walkers
+// hold few chains at a time, so they lose where the chip would be full with
+// a thread each, the more so the longer the traces (fewer of them fit a
+// block) and the higher the order; and short traces leave nothing to share
+// out.  Measured over traces of 8 to 15000 samples, 64 to 200000 chains and
+// orders 1 to 4 (blocks' gain over one thread each, one spray): order 2,
+// 128 x 2000 chains 1.71, 48 x 4000 0.59, 96 x 8000 1.00, 1000 x 20000 1.04,
+// 1000 x 80000 0.76, 2000 x 8000 1.26, 3000 x 20000 0.58, 8000 x 4000 1.11,
+// 8000 x 8000 0.69; order 3, 1000 x 8000 1.55, 1000 x 20000 0.65; order 4,
+// 2000 x 2000 1.22, 2000 x 8000 0.49.  The lines run where it is about 1.
+bool chain2_fits(int n1, int n2, int n3, int order, int sprays) {
+    const long slices = (long)n3 * sprays;
+    const double chains = 2.0 * n2 * slices;
+    if (n1 < (chains > 2048 ? 96 : order == 1 ? 48 : 32)) return false;
+    if (chains >= (order <= 3 ? 2000.0 : 1000.0) + (order <= 2 ? 18e6 : order == 3 ? 8e6 : 5e6) / n1) return false;
+    // (a slice's factor rows are addressed with 32-bit offsets)
+    return n3 <= 65535 && (double)n1 * n2 * 8 * order < 4294967295.0 && chain_plan(n1, n2, slices, order).nt > 0;
 }
 
 int chain2_factor(sh_ctx *ctx, const Pwsmooth2 &P) {

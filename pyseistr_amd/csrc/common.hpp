@@ -356,12 +356,13 @@ struct Pwsmooth2 {
     // (nullable) device flag: when it reads non-zero the spray kernels
     // return at once (a solver that has stopped)
     const int *stop = nullptr;
+    int sprays = 1;     // inputs sprayed in one launch (2: with the ones)
 };
-// The spray chains of P by blocks of threads (chain2.hip): whether its
-// traces fit, the factors of its slopes, the sprays of x into P.U (and of x2 into U2), and the adjoint
-// chains into P.C from the slots U or, with ww, from the field U weighted by
-// ww and the slots' weights.
-bool chain2_fits(int n1, int n2, int n3, int order);
+// The spray chains of P by blocks of threads (chain2.hip): whether they run
+// there, the factors of its slopes, the sprays of x into P.U (and of x2 into
+// U2), and the adjoint chains into P.C from the slots U or, with ww, from the
+// field U weighted by ww and the slots' weights.
+bool chain2_fits(int n1, int n2, int n3, int order, int sprays);
 int chain2_factor(sh_ctx *ctx, const Pwsmooth2 &P);
 int chain2_forward(sh_ctx *ctx, const Pwsmooth2 &P, const float *x, const float *x2, float *U2);
 int chain2_adjoint(sh_ctx *ctx, const Pwsmooth2 &P, const float *U, const float *ww);

@@ -1007,12 +1007,13 @@ bool spray2_buf(int n1, long n, int ns, int order, long nthr) {
         }                                    \
     } while (0)
 
-// The chains run by blocks of threads (chain2.hip) where a trace fits
-// their LDS, by one thread each otherwise; the switches of the
-// one-thread-per-chain kernels select those.
+// The chains run by blocks of threads (chain2.hip) where those fit and are
+// the faster, by one thread each otherwise; the switches of the
+// one-thread-per-chain kernels select those.  The same answer for the
+// factors, the sprays and the adjoint of one P.
 bool spray2_blocks(const Pwsmooth2 &P) {
     return !getenv("SH_SPRAY2_PF") && !getenv("SH_SPRAY2_BUF") && !getenv("SH_SPRAY2_TB") &&
-           chain2_fits(P.n1, P.n2, P.n3, P.order);
+           chain2_fits(P.n1, P.n2, P.n3, P.order, P.sprays);
 }
 
 // Factor cache of P into caller-provided buffers: scr holds 2*nthr*n1
@@ -1118,6 +1119,7 @@ int pws2_setup_forward(sh_ctx *ctx, Pwsmooth2 &P, int slot_base, const float *x,
     float *U1 = b + (long)ns2 * n;
     P.ww = b + (long)(2 * ns2) * n;
     P.C = b + (long)(2 * ns2 + 1) * n;
+    P.sprays = 2;
     SH_TRY(pws2_prepare(ctx, P, slot_base + 1, slot_base + 2));
     float *ones = P.C;
     int g = ceil_div(n, TB);
@@ -1489,7 +1491,8 @@ int somf2d_args(sh_ctx *ctx, const float *dn, const float *dip, const float *out
 // Workspace of one somf2d call, in floats, each part a multiple of 64
 // floats (256 bytes): staged data, dip and result (3n), the spray (n*np),
 // the chains' solver scratch (2*nthr*n1) and the factor cache
-// (2*(2*order+1)*n).
+// (3*(2*order+1)*n).  Scratch and the cache's last plane are the
+// one-thread-per-chain kernels'; the block kernels leave them alone.
 struct Somf2dWs {
     size_t b, U, scr, F, total;
 };

@@ -159,7 +159,8 @@ def test_chain_blocks_equal_single_threads(ps, monkeypatch, n1, n2, n3, ns, orde
         same(x, y, f"call {k}")
 
 
-@pytest.mark.parametrize("n1,n2,order", [(8, 1, 1), (9, 3, 2), (30, 40, 3), (21, 17, 4), (33, 70, 2), (65, 8, 2), (515, 9, 2)])
+@pytest.mark.parametrize("n1,n2,order", [(48, 1, 1), (49, 3, 1), (32, 40, 3), (35, 17, 4), (33, 70, 2), (65, 8, 2),
+                                         (515, 9, 2), (97, 1100, 2)])
 def test_chain_blocks_take_nothing_past_the_factors(ps, monkeypatch, n1, n2, order):
     """The block chains read whole groups of factor rows, past a trace's last
     one where its length is no multiple: with NaN all over the workspace
@@ -190,7 +191,7 @@ def test_chain_blocks_take_nothing_past_the_factors(ps, monkeypatch, n1, n2, ord
         same(a, b, f"call {k}")
 
 
-@pytest.mark.parametrize("n1,n2,order", [(15000, 600, 2), (15150, 513, 1), (14600, 1024, 3), (14400, 700, 4), (15000, 3, 2),
+@pytest.mark.parametrize("n1,n2,order", [(15000, 600, 2), (15150, 513, 1), (14600, 1024, 3), (14400, 600, 4), (15000, 3, 2),
                                          (15352, 2, 1), (16000, 2, 1), (130, 1100, 2), (300, 1100, 1)])
 def test_chain_block_limits(ps, monkeypatch, n1, n2, order):
     """The longest traces that blocks of chains hold, with one spray and with
