@@ -22,8 +22,12 @@ struct PGeo {
 // Blocks are dealt to the eight XCDs in turn; block b takes patch
 // (b % 8) * per + b / 8, so each XCD works through a contiguous run of patch
 // numbers and the overlapping neighbours share its L2.  Bound by writing the
-// patches; a plane's eight samples in flight instead of one: the section
-// below 175 -> 150 us (non-temporal stores 161).
+// patches.  PLANE: a 2-D patch's samples, eight of a thread in flight instead
+// of one (patches of at least four a thread; below, most of the eight would
+// repeat the last sample): 6000 x 2500 in patches of 256 x 128 192 -> 165 us,
+// 32 x 32 185 -> 179, but 16 x 32 207 -> 224.  A kernel of its own, as its
+// registers cost the other one 3 to 6 %.
+template <bool PLANE>
 __global__ void patch_cut(const double *__restrict__ in, double *__restrict__ X, PGeo g, long L, int npatch,
                           int per, FastDiv d1) {
     const int pid = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
@@ -34,7 +38,7 @@ __global__ void patch_cut(const double *__restrict__ in, double *__restrict__ X,
     const long n12 = (long)g.n[0] * g.n[1];
     const int m3 = min(l3, g.n[2] - b3);  // axis-3 samples inside the volume (may be <= 0)
     double *row = X + (long)pid * L;
-    if (l3 == 1) {  // a plane: eight of the thread's samples in flight
+    if constexpr (PLANE) {
         constexpr int U = 8;
         const double *src = in + n12 * min(b3, g.n[2] - 1);
         for (long q0 = threadIdx.x; q0 < l12; q0 += U * blockDim.x) {
@@ -83,11 +87,12 @@ __device__ inline void covering(int i, int l, int s, int P, int &lo, int &hi) {
 // One block per (i2, i3) column of the output, threads along i1.  Every
 // sample adds its covering patches in patch order (p1, then p2, then p3),
 // the order in which the reference accumulates them.  Bound by reading X,
-// each value once, U samples of a thread at a time (as many as a
-// trace gives 256 threads, up to four).  6000 x 2500 in patches of 256 x 128,
-// half overlapping (0.48 GB of patches): 167 us with one load in flight, 137
-// with four, 115 non-temporal (the copy's rate takes 128 us); 512 x 256 x 256
-// in 64 x 32 x 32: 430 -> 358.
+// each value once, U samples of a thread at a time (as many as a trace gives
+// 256 threads, up to four; patches shorter than 32 samples one, whose loads
+// are scattered already).  6000 x 2500 in half-overlapping patches of 256 x
+// 128 (0.48 GB): 157 us with one load in flight, 124 with four, 114
+// non-temporal (the copy's rate takes 128 us); of 12 x 12 201 with one, 242
+// with four, 329 non-temporal; 512 x 256 x 256 in 64 x 32 x 32: 430 -> 358.
 template <int U, bool NT>
 __global__ void patch_paste(const double *__restrict__ X, double *__restrict__ out, PGeo g, long L) {
     const int c = blockIdx.x;
@@ -177,8 +182,12 @@ extern "C" int sh_patch(sh_ctx *ctx, const double *in, double *X, int n1, int n2
     SH_TRY(geometry(ctx, n1, n2, n3, l1, l2, l3, s1, s2, s3, g, np, L));
     const int tpb = (int)std::min<long>(256, ceil_div((long)l1 * l2, 64) * 64);
     const int per = (int)ceil_div(np, 8);
-    hipLaunchKernelGGL(patch_cut, dim3((unsigned)(8L * per)), dim3(tpb), 0, ctx->stream, in, X, g, L, (int)np, per,
-                       FastDiv((unsigned)l1));
+    if (l3 == 1 && L >= 4 * 256)
+        hipLaunchKernelGGL(patch_cut<true>, dim3((unsigned)(8L * per)), dim3(tpb), 0, ctx->stream, in, X, g, L, (int)np,
+                           per, FastDiv((unsigned)l1));
+    else
+        hipLaunchKernelGGL(patch_cut<false>, dim3((unsigned)(8L * per)), dim3(tpb), 0, ctx->stream, in, X, g, L, (int)np,
+                           per, FastDiv((unsigned)l1));
     return sh_launch_check(ctx, "patch_cut");
 }
 
@@ -193,10 +202,13 @@ extern "C" int sh_patch_inv(sh_ctx *ctx, const double *X, double *out, int n1, i
     const dim3 grid((unsigned)((long)n2 * n3));
     // non-temporal where the patches are more than the Infinity Cache holds
     // (200 x 100 x 100 in half-overlapping cubes of 32: 41 us, plain loads 32)
-    const bool nt = (size_t)np * L * sizeof(double) > (256u << 20);
+    // and their rows begin and end with a 128-byte line: the samples of a
+    // shared line are read in different turns (6000 x 2500 in 48 x 48, step
+    // 24: 153 us, plain loads 139; 32 x 32, step 16: 122 and 134)
+    const bool nt = (size_t)np * L * sizeof(double) > (256u << 20) && l1 % 16 == 0 && s1 % 16 == 0;
 #define PP_(U, N) hipLaunchKernelGGL((patch_paste<U, N>), grid, dim3(tpb), 0, ctx->stream, X, out, g, L)
-    if (n1 > 3 * 256) { if (nt) PP_(4, true); else PP_(4, false); }
-    else if (n1 > 384) { if (nt) PP_(2, true); else PP_(2, false); }
+    if (l1 >= 32 && n1 > 3 * 256) { if (nt) PP_(4, true); else PP_(4, false); }
+    else if (l1 >= 32 && n1 > 384) { if (nt) PP_(2, true); else PP_(2, false); }
     else { if (nt) PP_(1, true); else PP_(1, false); }
 #undef PP_
     return sh_launch_check(ctx, "patch_paste");

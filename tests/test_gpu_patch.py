@@ -56,6 +56,19 @@ def test_batches_of_a_thread_bit_exact(pm, n, l, s):
     assert np.array_equal(pm.patch2d_inv(Y, *n, *l, *s), P.paste(Y, n, l, s), equal_nan=True)
 
 
+@pytest.mark.parametrize("l,s", [((31, 33), (16, 16)), ((32, 32), (16, 16)), ((16, 64), (16, 20)), ((31, 40), (9, 40)),
+                                 ((33, 31), (17, 16)), ((48, 24), (24, 12))])
+def test_patch_size_rules_bit_exact(pm, l, s):
+    """Planes of 1023 and 1024 samples (one a time, or eight of a thread in
+    flight) and patches a sample shorter and longer than 32 (one sample of a
+    thread's trace at a time, or up to four)."""
+    A = np.random.default_rng(l[0]).standard_normal((1200, 75))
+    X = pm.patch2d(A, *l, *s)
+    assert np.array_equal(X, P.cut(A, l, s))
+    Y = np.random.default_rng(l[1]).standard_normal(X.shape)
+    assert np.array_equal(pm.patch2d_inv(Y, 1200, 75, *l, *s), P.paste(Y, (1200, 75), l, s), equal_nan=True)
+
+
 @pytest.mark.parametrize("pad", list(itertools.product([0, 1], repeat=3)))
 def test_patch3d_every_padding_case(pm, pad):
     # l = (6, 4, 4), s = (3, 2, 2): n fits exactly when (n - l) % s == 0
