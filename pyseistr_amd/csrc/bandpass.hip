@@ -127,7 +127,9 @@ int cascade_of(const Butter &bw, Cascade &c, int ns) {
 // wave a SIMD), 8 instructions a section and sample; with one wave doing
 // both, each chunk waited for its loads besides: 500 samples of 37500 traces,
 // two sections, 128 -> 36 us a pass.  The first pass reads its input where
-// it is.
+// it is.  Traces of one chunk stream nothing: both waves move it in and out,
+// in half the LDS, so twice the blocks are on a CU (1000000 traces of 20
+// samples, two sections, four passes: 339 us streamed, 178 so).
 //
 // ODD0: the first section is of odd order (its filter's own).  MIX: so may a
 // later one be (both filters in one pass).  A section's sign of the high or
@@ -166,7 +168,8 @@ constexpr int BP_C = 64;  // traces of a block, samples of a chunk
 template <int NS, bool ODD0, bool MIX>
 __global__ void __launch_bounds__(2 * BP_C)
 bandpass_fused(const float *in, float *out, long ntr, int n1, const Cascade c, int back) {
-    __shared__ float tile[2][BP_C][BP_C + 1];
+    extern __shared__ float bp_lds[];  // one chunk, or two in turn
+    float (*const tile)[BP_C][BP_C + 1] = reinterpret_cast<float (*)[BP_C][BP_C + 1]>(bp_lds);
     const int t = threadIdx.x % BP_C;
     const bool walks = threadIdx.x < BP_C;
     const long tr0 = (long)blockIdx.x * BP_C;
@@ -193,10 +196,26 @@ bandpass_fused(const float *in, float *out, long ntr, int n1, const Cascade c, i
 #pragma unroll 16
         for (int r = 0; r < nr; r++) p[(long)r * n1] = src[t][r];
     };
+    if (nch == 1) {  // short traces: nothing to stream, both waves move them
+        const int r0 = walks ? 0 : BP_C / 2, r1 = min(nr, r0 + BP_C / 2);
+        if (t < n1)
+#pragma unroll 8
+            for (int r = r0; r < r1; r++) tile[0][t][r] = in[(tr0 + r) * n1 + t];
+        __syncthreads();
+        if (walks) {
+            float *p = &tile[0][back ? n1 - 1 : 0][t];
+            for (int kk = 0; kk < n1; kk++, p += back ? -(BP_C + 1) : BP_C + 1) *p = w.step(c, *p);
+        }
+        __syncthreads();
+        if (t < n1)
+#pragma unroll 8
+            for (int r = r0; r < r1; r++) out[(tr0 + r) * n1 + t] = tile[0][t][r];
+        return;
+    }
     if (!walks) {
         load(0);
         put(tile[0]);
-        if (nch > 1) load(1);
+        load(1);
     }
     __syncthreads();
     for (int ci = 0; ci < nch; ci++) {
@@ -227,10 +246,11 @@ bandpass_fused(const float *in, float *out, long ntr, int n1, const Cascade c, i
 
 int launch_fused(sh_ctx *ctx, const float *in, float *out, long ntr, int n1, const Cascade &c, int ns, int back) {
     const dim3 grid((unsigned)ceil_div(ntr, BP_C)), block(2 * BP_C);
+    const size_t lds = sizeof(float) * BP_C * (BP_C + 1) * (n1 > BP_C ? 2 : 1);
     bool mix = false;
     for (int s = 1; s < ns; s++) mix = mix || c.st[s].odd;
     switch (ns) {
-#define BP_K(N, O, M) hipLaunchKernelGGL((bandpass_fused<N, O, M>), grid, block, 0, ctx->stream, in, out, ntr, n1, c, back)
+#define BP_K(N, O, M) hipLaunchKernelGGL((bandpass_fused<N, O, M>), grid, block, lds, ctx->stream, in, out, ntr, n1, c, back)
 #define BP_CASE(N)                                               \
     case N:                                                      \
         if (mix) { if (c.st[0].odd) BP_K(N, true, true); else BP_K(N, false, true); }   \
