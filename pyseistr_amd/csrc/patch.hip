@@ -22,13 +22,16 @@ struct PGeo {
 // Blocks are dealt to the eight XCDs in turn; block b takes patch
 // (b % 8) * per + b / 8, so each XCD works through a contiguous run of patch
 // numbers and the overlapping neighbours share its L2.  Bound by writing the
-// patches.  PLANE: a 2-D patch's samples, eight of a thread in flight instead
-// of one (patches of at least four a thread; below, most of the eight would
-// repeat the last sample): 6000 x 2500 in patches of 256 x 128 192 -> 165 us,
-// 32 x 32 185 -> 179, but 16 x 32 207 -> 224.  A kernel of its own, as its
-// registers cost the other one 3 to 6 %.
-template <bool PLANE>
-__global__ void patch_cut(const double *__restrict__ in, double *__restrict__ X, PGeo g, long L, int npatch,
+// patches.  WAVES > 0: a 2-D patch's samples, eight of a thread in flight
+// instead of one (patches of at least four a thread; below, most of the eight
+// would repeat the last sample): 6000 x 2500 in patches of 256 x 128 191 ->
+// 166 us, 32 x 32 185 -> 178, but 16 x 32 207 -> 224.  Kernels of their own,
+// as their registers cost the other one 3 to 6 %; and with WAVES of a SIMD at
+// a time: patches of 4096 samples or more take four, so that fewer are cut
+// side by side and the lines they share stay in the L2 (64 x 64 161 -> 143,
+// 256 x 128 166 -> 159, but 32 x 32 178 -> 190).
+template <int WAVES>
+__global__ void __attribute__((amdgpu_waves_per_eu(WAVES ? WAVES : 1, WAVES ? WAVES : 8))) patch_cut(const double *__restrict__ in, double *__restrict__ X, PGeo g, long L, int npatch,
                           int per, FastDiv d1) {
     const int pid = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
     if (pid >= npatch) return;
@@ -38,7 +41,7 @@ __global__ void patch_cut(const double *__restrict__ in, double *__restrict__ X,
     const long n12 = (long)g.n[0] * g.n[1];
     const int m3 = min(l3, g.n[2] - b3);  // axis-3 samples inside the volume (may be <= 0)
     double *row = X + (long)pid * L;
-    if constexpr (PLANE) {
+    if constexpr (WAVES > 0) {
         constexpr int U = 8;
         const double *src = in + n12 * min(b3, g.n[2] - 1);
         for (long q0 = threadIdx.x; q0 < l12; q0 += U * blockDim.x) {
@@ -182,12 +185,13 @@ extern "C" int sh_patch(sh_ctx *ctx, const double *in, double *X, int n1, int n2
     SH_TRY(geometry(ctx, n1, n2, n3, l1, l2, l3, s1, s2, s3, g, np, L));
     const int tpb = (int)std::min<long>(256, ceil_div((long)l1 * l2, 64) * 64);
     const int per = (int)ceil_div(np, 8);
-    if (l3 == 1 && L >= 4 * 256)
-        hipLaunchKernelGGL(patch_cut<true>, dim3((unsigned)(8L * per)), dim3(tpb), 0, ctx->stream, in, X, g, L, (int)np,
-                           per, FastDiv((unsigned)l1));
-    else
-        hipLaunchKernelGGL(patch_cut<false>, dim3((unsigned)(8L * per)), dim3(tpb), 0, ctx->stream, in, X, g, L, (int)np,
-                           per, FastDiv((unsigned)l1));
+#define PC_(W)                                                                                                       \
+    hipLaunchKernelGGL(patch_cut<W>, dim3((unsigned)(8L * per)), dim3(tpb), 0, ctx->stream, in, X, g, L, (int)np, per, \
+                       FastDiv((unsigned)l1))
+    if (l3 == 1 && L >= 4096) PC_(4);
+    else if (l3 == 1 && L >= 1024) PC_(8);
+    else PC_(0);
+#undef PC_
     return sh_launch_check(ctx, "patch_cut");
 }
 

@@ -57,10 +57,10 @@ def test_batches_of_a_thread_bit_exact(pm, n, l, s):
 
 
 @pytest.mark.parametrize("l,s", [((31, 33), (16, 16)), ((32, 32), (16, 16)), ((16, 64), (16, 20)), ((31, 40), (9, 40)),
-                                 ((33, 31), (17, 16)), ((48, 24), (24, 12))])
+                                 ((33, 31), (17, 16)), ((48, 24), (24, 12)), ((65, 63), (33, 32)), ((64, 64), (32, 64))])
 def test_patch_size_rules_bit_exact(pm, l, s):
     """Planes of 1023 and 1024 samples (one a time, or eight of a thread in
-    flight) and patches a sample shorter and longer than 32 (one sample of a
+    flight), of 4095 and 4096 (fewer waves at a time), and patches a sample shorter and longer than 32 (one sample of a
     thread's trace at a time, or up to four)."""
     A = np.random.default_rng(l[0]).standard_normal((1200, 75))
     X = pm.patch2d(A, *l, *s)
