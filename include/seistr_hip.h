@@ -68,7 +68,8 @@ int sh_ctx_trim(sh_ctx *ctx);
 int sh_c_to_f(sh_ctx *ctx, const float *in, float *out, int n1, int n2, int n3);
 const char *sh_last_error(const sh_ctx *ctx);
 int sh_version(void);
-/* Block until all work queued on the context's stream has finished. */
+/* Block until all work queued on the context's stream has finished.  SH_EHIP
+ * also if an earlier sh_dip of a 2-D section failed on the device. */
 int sh_sync(sh_ctx *ctx);
 
 /* Launch timing (no counterpart in the reference; instrumentation for the
@@ -100,6 +101,10 @@ typedef struct {
  * idip/xdip inputs, dip_cfuns.c:1861-1875).  eps_dv is accepted and has no
  * effect, as in the reference (its shared `eps` static is reset to 1).
  * rep (nullable, host memory): iteration record; filling it synchronises.
+ * A 2-D section that fits the chip runs as one launch whose blocks wait for
+ * each other; should one not arrive within seconds, the dips are NaN and the
+ * call, where it synchronises, or else the next sh_sync or sh_dip returns
+ * SH_EHIP.
  * With n3 > 1 the two directions are independent: the crossline one runs
  * on a second stream owned by the context, forked from and joined back to
  * the context's stream inside the call, so every result is ordered on the

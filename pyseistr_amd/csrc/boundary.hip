@@ -181,6 +181,7 @@ int sh_dip(sh_ctx *ctx, const float *data, const float *mask, const float *init,
     if (!data || !dip) return sh_fail(ctx, SH_ENULL, "sh_dip: data and dip must be non-NULL");
     if (n1 < 1 || n2 < 1 || n3 < 1) return sh_fail(ctx, SH_EINVAL, "sh_dip: bad shape %d x %d x %d", n1, n2, n3);
     const long n = (long)n1 * n2 * n3, nd = n3 == 1 ? n : 2 * n;
+    SH_TRY(sh_wait_status(ctx));  // an earlier estimate that was not waited for
     Boundary B(ctx, "sh_dip");
     SH_IN(B, data, n);
     SH_IN(B, mask, n);
@@ -200,7 +201,8 @@ int sh_dip(sh_ctx *ctx, const float *data, const float *mask, const float *init,
         SH_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev_t0, ctx->ev_t1));
         rep->elapsed_ms = ms;
     }
-    return B.finish(rc);
+    SH_TRY(B.finish(rc));
+    return ctx->flags & SH_FLAG_HOST_PTRS ? sh_wait_status(ctx) : SH_OK;
 }
 
 int sh_pwspray3d(sh_ctx *ctx, const float *din, const float *dipi, const float *dipx, int n1, int n2, int n3,

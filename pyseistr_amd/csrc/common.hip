@@ -45,6 +45,11 @@ int sh_launch_check(sh_ctx *ctx, const char *what) {
     return SH_OK;
 }
 
+int sh_wait_status(sh_ctx *ctx) {
+    if (!ctx->wait_failed || !__atomic_exchange_n(ctx->wait_failed, 0, __ATOMIC_ACQ_REL)) return SH_OK;
+    return sh_fail(ctx, SH_EHIP, "sh_dip: the blocks of a 2-D section did not meet; its dips are NaN");
+}
+
 __global__ void __launch_bounds__(1024) reduce_partials_kernel(const double *part, int nblk, int K, double *out) {
     __shared__ double sh[16];
     for (int k = 0; k < K; k++) {
@@ -179,6 +184,7 @@ void sh_ctx_destroy(sh_ctx *ctx) {
     if (ctx->ev_t0) (void)hipEventDestroy(ctx->ev_t0);
     if (ctx->ev_t1) (void)hipEventDestroy(ctx->ev_t1);
     if (ctx->ev_switch) (void)hipEventDestroy(ctx->ev_switch);
+    if (ctx->wait_failed) (void)hipHostFree(ctx->wait_failed);
     if (ctx->aux) {
         (void)hipStreamDestroy(ctx->aux);
         (void)hipEventDestroy(ctx->ev_fork);
@@ -209,7 +215,7 @@ int sh_version(void) { return 100; }
 int sh_sync(sh_ctx *ctx) {
     if (!ctx) return SH_ENULL;
     SH_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return SH_OK;
+    return sh_wait_status(ctx);
 }
 
 }  // extern "C"

@@ -47,6 +47,9 @@ struct sh_ctx {
     // the deleter destroys them)
     std::shared_ptr<void> fk;
     std::shared_ptr<void> fk_tables;
+    // set by a kernel whose blocks did not meet at their barrier (pinned host
+    // memory, made with the first such kernel): sh_wait_status
+    int *wait_failed = nullptr;
     // SH_FLAG_* of the public entry points (sh_ctx_set_flags)
     int flags = 0;
     // brackets of a dip call's device time (sh_dip_report.elapsed_ms)
@@ -84,6 +87,10 @@ int sh_slot(sh_ctx *ctx, int id, size_t bytes, void **out);
 
 // Launch-error check after a kernel launch.
 int sh_launch_check(sh_ctx *ctx, const char *what);
+
+// SH_EHIP if a barrier of an earlier call failed (and clears that); a call
+// that has not run yet is seen after a synchronisation only.
+int sh_wait_status(sh_ctx *ctx);
 
 // Slot ids (each module owns a range so that nested calls do not collide).
 enum {

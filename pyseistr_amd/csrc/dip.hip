@@ -1152,6 +1152,7 @@ extern "C" int shd_dip(sh_ctx *ctx, const float *data, const float *mask, const 
                 rep->niter = niter;
                 SH_HIP(ctx, hipMemcpyAsync(h, rec, sizeof h, hipMemcpyDeviceToHost, ctx->stream));
                 SH_HIP(ctx, hipStreamSynchronize(ctx->stream));
+                SH_TRY(sh_wait_status(ctx));
                 for (int it = 0; it < niter && it < 64; it++) {
                     rep->cg_iters[0][it] = h[2 * it];
                     rep->ls_step[0][it] = h[2 * it + 1];

@@ -25,8 +25,13 @@
 // Every block adds up all sums in the same order and keeps its own copy of
 // the scalar record, so all take the same decisions.  The launch is
 // cooperative, so all blocks are on the chip at once; the wait is bounded all
-// the same, and a block that gives up fills its dips with NaN.
+// the same, and a block that gives up fills its dips with NaN and sets the
+// context's flag, which the next call that synchronises (or the next
+// estimate) turns into an error.
 #include "dip2.hpp"
+
+#include <algorithm>
+#include <cstdlib>
 
 namespace {
 
@@ -45,6 +50,8 @@ struct Resident {
     unsigned long long *words;  // [2][blocks][2 * LS_SUMS]
     float *dip;
     int *rec;
+    int polls;    // before a block gives up
+    int *failed;  // set then (host memory)
 };
 
 // Element i of a section's field.  The index is hidden from the optimiser
@@ -82,9 +89,9 @@ __device__ inline bool meet(const Resident &R, unsigned epoch, double (&v)[K], d
             __hip_atomic_store(w + 1, tag | (b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     if (threadIdx.x < 64) {
-        double s[K];
+        double s[K] = {};
         bool all = false;
-        for (int n = 0; n < WAIT_MAX && !all; n++) {
+        for (int n = 0; n < R.polls && !all; n++) {
             bool here = true;
 #pragma unroll
             for (int k = 0; k < K; k++) s[k] = 0.0;
@@ -366,6 +373,7 @@ d2_resident(const Resident R) {
 #pragma unroll
     for (int j = 0; j < 4; j++)
         if (mine(j)) R.dip[o0 + j * n1] = fine ? p[j] : __builtin_nanf("");
+    if (!fine && tid == 0) __hip_atomic_store(R.failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (R.rec && blockIdx.x == 0)
         for (int q = tid; q < 2 * min(R.niter, 64); q += TBR) R.rec[q] = s.rec[q];
 }
@@ -416,7 +424,18 @@ int dip2_resident(sh_ctx *ctx, int n1, int n2, int r1, int r2, int order, const 
     const int nb = tiles_of(c, n1, n2), he = held_of(c, r1, r2);
     const void *fn = nullptr;
     SH_DISPATCH_NW6(ctx, order, NW, fn = he == 9 ? res_kernel<NW, 9>(c) : res_kernel<NW, 16>(c));
-    Resident R{n1, n2, r1, r2, niter, liter, x, init, mask, nullptr, nullptr, dip, rec};
+    if (!ctx->wait_failed) {
+        const hipError_t e = hipHostMalloc((void **)&ctx->wait_failed, sizeof(int), hipHostMallocDefault);
+        if (e != hipSuccess) {
+            ctx->wait_failed = nullptr;
+            return sh_fail(ctx, SH_EALLOC, "hipHostMalloc: %s", hipGetErrorString(e));
+        }
+        *ctx->wait_failed = 0;
+    }
+    // SH_DIP2_POLLS: fewer polls (0: give up at the first barrier)
+    const char *pe = getenv("SH_DIP2_POLLS");
+    const int polls = pe ? std::min(std::max(atoi(pe), 0), WAIT_MAX) : WAIT_MAX;
+    Resident R{n1, n2, r1, r2, niter, liter, x, init, mask, nullptr, nullptr, dip, rec, polls, ctx->wait_failed};
     SH_TRY(sh_slot(ctx, SLOT_DIP0, (size_t)n * 3 * sizeof(float), (void **)&R.ex));
     const size_t nw = (size_t)2 * nb * 2 * LS_SUMS;
     SH_TRY(sh_slot(ctx, SLOT_RED, nw * sizeof(unsigned long long), (void **)&R.words));

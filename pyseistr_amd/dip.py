@@ -60,7 +60,11 @@ def _run(din, shape, niter, liter, order, eps_dv, rect, mask, init, report):
     res = dip_device(d, shape, niter, liter, order, eps_dv, rect, m, ini, report=report)
     if report:
         return _lib.to_host(res[0]), res[1]
-    return _lib.to_host(res)
+    res = _lib.to_host(res)
+    if shape[2] == 1:  # the copy has waited for the section; this asks how it went
+        ctx = _lib.context()
+        _lib.check(ctx, _lib.load().sh_sync(ctx), "dip")
+    return res
 
 
 def dip2dc(din, niter=5, liter=20, order=2, eps_dv=0.01, eps_cg=1, tol_cg=0.000001, rect=[10, 10, 1], verb=1,

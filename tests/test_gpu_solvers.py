@@ -370,3 +370,41 @@ def test_resident_sections_from_threads(ps):
     buf = data[1].clone()
     dip.dip_device(buf, shapes[1], niter=2, rect=(6, 6, 1), out=buf)
     assert np.array_equal(buf.cpu().numpy(), alone[1])
+
+
+def test_section_whose_blocks_do_not_meet_is_an_error(ps, monkeypatch):
+    """With no polls allowed (SH_DIP2_POLLS=0) every block of a section gives
+    up at its first barrier: NaN dips, and an error from the call where it
+    waits (drop-in, report, host pointers), else from the next sh_sync or
+    estimate, once.  The estimates after it are as before."""
+    import ctypes
+
+    import torch
+    from pyseistr_amd import _lib, dip
+    shape = (130, 70, 1)
+    d = np.random.default_rng(9).standard_normal(shape[:2]).astype(np.float32)
+    x = _lib.to_device(d)
+    kw = dict(niter=2, liter=6, rect=(6, 6, 1))
+    good = dip.dip_device(x, shape, **kw).cpu().numpy()
+    lib, ctx = _lib.load(), _lib.context()
+    flat, out = F(d), np.empty(good.size, np.float32)
+    args = [ctx, flat.ctypes.data_as(ctypes.c_void_p), None, None, *shape, 2, 6, 2, 0.01, 6, 6, 1,
+            out.ctypes.data_as(ctypes.c_void_p), None]
+    monkeypatch.setenv("SH_DIP2_POLLS", "0")
+    with pytest.raises(_lib.SeistrError, match="did not meet"):
+        ps.dip2dc(d, niter=2, liter=6, rect=[6, 6, 1])
+    with pytest.raises(_lib.SeistrError, match="did not meet"):
+        ps.dip2dc(d, niter=2, liter=6, rect=[6, 6, 1], report=True)
+    assert lib.sh_ctx_set_flags(ctx, _lib.FLAG_HOST_PTRS) == 0
+    rc = lib.sh_dip(*args)
+    assert lib.sh_ctx_set_flags(ctx, 0) == 0
+    assert rc == -4 and np.isnan(out).all()
+    assert torch.isnan(dip.dip_device(x, shape, **kw)).all()
+    assert lib.sh_sync(ctx) == -4 and lib.sh_sync(ctx) == 0
+    dip.dip_device(x, shape, **kw)
+    torch.cuda.synchronize()
+    monkeypatch.delenv("SH_DIP2_POLLS")
+    with pytest.raises(_lib.SeistrError, match="did not meet"):
+        dip.dip_device(x, shape, **kw)
+    assert np.array_equal(dip.dip_device(x, shape, **kw).cpu().numpy(), good)
+    assert lib.sh_sync(ctx) == 0
