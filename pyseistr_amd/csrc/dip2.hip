@@ -445,12 +445,15 @@ int dip2_resident(sh_ctx *ctx, int n1, int n2, int r1, int r2, int order, const 
     PROF_A(ctx);
     const hipError_t e = hipLaunchCooperativeKernel(fn, dim3(nb), dim3(TBR), args,
                                                     (unsigned)res_lds(T_CFG[c][0], T_CFG[c][1], r1, r2), ctx->stream);
-    // the three exchanged fields of an iteration, written and read
-    PROF_B(ctx, "d2_resident", 24.0 * (double)n * niter * liter);
-    if (e != hipSuccess) {  // the device does not take it: nothing was started
+    if (e != hipSuccess) {
         (void)hipGetLastError();
-        return SH_OK;
+        // more blocks than this device holds at once, or none of the kind: the launches run
+        if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported) return SH_OK;
+        return sh_fail(ctx, SH_EHIP, "launch of d2_resident failed: %s", hipGetErrorString(e));
     }
+    // the three exchanged fields of an iteration, written and read, if every
+    // solve takes all its iterations
+    PROF_B(ctx, "d2_resident", 24.0 * (double)n * niter * liter);
     *ran = 1;
     return SH_OK;
 }
