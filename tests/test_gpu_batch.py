@@ -124,6 +124,26 @@ def test_batch_workspace_reuse_and_gaps(env):
     assert np.array_equal(_bits(whole), _bits(np.concatenate([u.ravel(order="F") for u in first])))
 
 
+def test_batch_after_a_batch_of_nan(env):
+    """Fields and partial sums of a batch left full of NaN by one before it
+    (its data NaN) reach nothing: the dips, their record and the filtered
+    patches have the bits they have first, one patch all zeros among them
+    (its solves end before they begin)."""
+    batch, pats = env
+    pats = [p for p in pats[:3]] + [np.zeros((40, 30), np.float32)]
+    b = batch.Batch(pats)
+    first, rec = batch.dip2d_batched(b, niter=3, liter=6, report=True)
+    first = first.clone()
+    med = batch.somf2d_batched(b, first, ns=5).clone()
+    big = batch.Batch([np.full((p.shape[0] + 40, p.shape[1] + 20), np.nan, np.float32) for p in pats])
+    bad = batch.dip2d_batched(big, niter=3, liter=6)
+    assert np.isnan(bad.cpu().numpy()).any()
+    batch.somf2d_batched(big, bad, ns=5)
+    again, rec2 = batch.dip2d_batched(b, niter=3, liter=6, report=True)
+    assert np.array_equal(_bits(first.cpu().numpy()), _bits(again.cpu().numpy())) and np.array_equal(rec, rec2)
+    assert np.array_equal(_bits(med.cpu().numpy()), _bits(batch.somf2d_batched(b, again, ns=5).cpu().numpy()))
+
+
 def test_dip2d_batched_against_oracle(env):
     from oracle import oracle as O
     batch, pats = env
