@@ -483,12 +483,20 @@ int bdip(sh_ctx *ctx, const BatchTables &T, int cfg, int r1, int r2, const float
         const float pmax = 3.402823466e+38f, pmin = -3.402823466e+38f;
         SH_TRY(bpwd_launch<NW>(ctx, T, 2, x, W.p[cur], W.dp, 1.0f, W.p[1 - cur], W));
         SH_TRY(bfin(ctx, T, W, 1, 0, F_LS0, it));
-        hipLaunchKernelGGL((bhalved<NW>), g, dim3(TB), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax, T.P, T.blk_patch,
-                           W.part, T.nblk, W.sc);
+        {
+            PROF_A(ctx);
+            hipLaunchKernelGGL((bhalved<NW>), g, dim3(TB), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax, T.P,
+                               T.blk_patch, W.part, T.nblk, W.sc);
+            PROF_B(ctx, "bhalved", 12.0 * (double)T.ntot);
+        }
         SH_TRY(sh_launch_check(ctx, "bhalved"));
         SH_TRY(bfin(ctx, T, W, LS_SUMS, 0, F_LS7, it));
-        hipLaunchKernelGGL((bchosen<NW>), g, dim3(TB), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax, W.p[1 - cur], W.u2,
-                           T.P, T.blk_patch, W.sc);
+        {
+            PROF_A(ctx);
+            hipLaunchKernelGGL((bchosen<NW>), g, dim3(TB), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax, W.p[1 - cur],
+                               W.u2, T.P, T.blk_patch, W.sc);
+            PROF_B(ctx, "bchosen", 20.0 * (double)T.ntot);
+        }
         SH_TRY(sh_launch_check(ctx, "bchosen"));
         cur = 1 - cur;
     }

@@ -890,7 +890,8 @@ int smooth_apply(sh_ctx *ctx, const DipGeom &g, const SmoothPlan &sp, const floa
         if (pro == PRO_CG) { if (nt) SM_P12(PRO_CG, true); else SM_P12(PRO_CG, false); }
         else { if (nt) SM_P12(PRO_PLAIN, true); else SM_P12(PRO_PLAIN, false); }
 #undef SM_P12
-        PROF_B(ctx, pro == PRO_CG ? "smooth_pair12<1>" : "smooth_pair12<0>",
+        PROF_B(ctx, pro == PRO_CG ? (nt ? "smooth_pair12<1,true>" : "smooth_pair12<1,false>")
+                                  : (nt ? "smooth_pair12<0,true>" : "smooth_pair12<0,false>"),
                pass_bytes(pro, EPI_PLAIN, first != 0, false) * (double)g.n);
         SH_TRY(sh_launch_check(ctx, "smooth_pair12"));
         src = W.t1;
@@ -1071,12 +1072,20 @@ int dip_direction(sh_ctx *ctx, const DipGeom &g, const SmoothPlan &plan, int axi
         SH_TRY(finalize(ctx, W, nb_pw, 1, F_LS0, it, n));
         const float pmax = 3.402823466e+38f, pmin = -3.402823466e+38f;
         const FastDiv f1((unsigned)g.n1), f2((unsigned)g.n2);
-        hipLaunchKernelGGL((pwd_halved<NW>), dim3(nb_pw), dim3(256), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax, g.n1,
-                           g.n2, g.n3, axis, W.part, W.sc, f1, f2);
+        {
+            PROF_A(ctx);
+            hipLaunchKernelGGL((pwd_halved<NW>), dim3(nb_pw), dim3(256), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax,
+                               g.n1, g.n2, g.n3, axis, W.part, W.sc, f1, f2);
+            PROF_B(ctx, "pwd_halved", 12.0 * (double)n);
+        }
         SH_TRY(sh_launch_check(ctx, "pwd_halved"));
         SH_TRY(finalize(ctx, W, nb_pw, LS_SUMS, F_LS7, it, n));
-        hipLaunchKernelGGL((pwd_chosen<NW>), dim3(nb_pw), dim3(256), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax,
-                           W.p[1 - cur], W.u2, g.n1, g.n2, g.n3, axis, W.sc, f1, f2);
+        {
+            PROF_A(ctx);
+            hipLaunchKernelGGL((pwd_chosen<NW>), dim3(nb_pw), dim3(256), 0, ctx->stream, x, W.p[cur], W.dp, pmin, pmax,
+                               W.p[1 - cur], W.u2, g.n1, g.n2, g.n3, axis, W.sc, f1, f2);
+            PROF_B(ctx, "pwd_chosen", 20.0 * (double)n);
+        }
         SH_TRY(sh_launch_check(ctx, "pwd_chosen"));
         cur = 1 - cur;
     }

@@ -763,12 +763,12 @@ int soint_solve(sh_ctx *ctx, const Geo &g0, const float *pp, const float *qq, co
         {
             PROF_A(ctx);
             SH_TRY(pwd_adj_launch<NW>(ctx, g, rr, known, gv, pa, nba, st));
-            PROF_B(ctx, "pwd_adj", 4.0 * (ny + g.nparts * n + n));
+            PROF_B(ctx, ranges ? "pwd_adj_range" : "pwd_adj", 4.0 * (ny + g.nparts * n + n));
         }
         {
             PROF_A(ctx);
             SH_TRY(pwd_fwd_launch<NW>(ctx, g, gv, gg, Ss, rr, part, nbf, nullptr, st));
-            PROF_B(ctx, "pwd_fwd", 4.0 * (n + g.nparts * n + 3 * ny));
+            PROF_B(ctx, ranges ? "pwd_fwd_range" : "pwd_fwd", 4.0 * (n + g.nparts * n + 3 * ny));
         }
         hipLaunchKernelGGL(cgstep_scalars, dim3(1), dim3(1024), 0, ctx->stream, pa, nba, part, nbf, st, 0);
         PROF_A(ctx);

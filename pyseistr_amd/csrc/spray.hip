@@ -1026,7 +1026,12 @@ int pws2_prepare_bufs(sh_ctx *ctx, Pwsmooth2 &P, float *scr, float *F) {
     P.scr = scr;
     P.tr = P.scr + (long)P.nthr * P.n1;
     P.F = F;
-    if (spray2_blocks(P)) return chain2_factor(ctx, P);
+    if (spray2_blocks(P)) {
+        PROF_A(ctx);
+        SH_TRY(chain2_factor(ctx, P));
+        PROF_B(ctx, "chain2_rows+ldl", 4.0 * (double)n);
+        return SH_OK;
+    }
     const int TB2 = spray2_tb();
     dim3 grid(ceil_div(2L * P.n2, TB2), P.n3);
     PROF_A(ctx);
@@ -1065,7 +1070,7 @@ int pws2_adjoint(sh_ctx *ctx, Pwsmooth2 &P, bool blocks, const float *U, const f
                        hipLaunchKernelGGL((spray2_adj<BUF, NW, PF>), grid, dim3(TB2), 0, ctx->stream, U, P.dip, P.F,
                                           P.C, P.n1, P.n2, P.n3, P.ns, P.e, P.scr, P.tr, P.nthr, P.stop))));
     }
-    PROF_B(ctx, "spray2_adj", 12.0 * 2 * P.ns * (double)n);
+    PROF_B(ctx, blocks ? "chain2_adj" : "spray2_adj", 12.0 * 2 * P.ns * (double)n);
     return sh_launch_check(ctx, "spray2_adj");
 }
 
@@ -1074,7 +1079,8 @@ int pws2_adjoint(sh_ctx *ctx, Pwsmooth2 &P, bool blocks, const float *U, const f
 // two latency-bound sets of chains run side by side.
 int pws2_spray(sh_ctx *ctx, Pwsmooth2 &P, const float *x, const float *x2 = nullptr, float *U2 = nullptr) {
     PROF_A(ctx);
-    if (spray2_blocks(P)) {
+    const bool blocks = spray2_blocks(P);
+    if (blocks) {
         SH_TRY(chain2_forward(ctx, P, x, x2, U2));
     } else {
         const int TB2 = spray2_tb();
@@ -1084,7 +1090,7 @@ int pws2_spray(sh_ctx *ctx, Pwsmooth2 &P, const float *x, const float *x2 = null
                        hipLaunchKernelGGL((spray2_fwd<BUF, NW, PF>), grid, dim3(TB2), 0, ctx->stream, x, P.dip, P.F,
                                           P.U, P.n1, P.n2, P.n3, P.ns, P.e, P.scr, P.nthr, P.stop, x2, U2))));
     }
-    PROF_B(ctx, "spray2_fwd", (x2 ? 2 : 1) * 12.0 * 2 * P.ns * (double)P.n1 * P.n2 * P.n3);
+    PROF_B(ctx, blocks ? "chain2_fwd" : "spray2_fwd", (x2 ? 2 : 1) * 12.0 * 2 * P.ns * (double)P.n1 * P.n2 * P.n3);
     return sh_launch_check(ctx, "spray2_fwd");
 }
 
