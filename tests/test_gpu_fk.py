@@ -71,6 +71,37 @@ def test_transform_lengths(fk, n1, n2):
         assert _rel(got, ref) <= TOL
 
 
+def _long_double(d, w):
+    """oracle.fk_oracle.fkdip in long double."""
+    n1, n2 = d.shape
+    nf, nk = F.nextpow2(n1), F.nextpow2(n2)
+    h = nf // 2 + 1
+    D = np.fft.fftshift(np.fft.fft(np.fft.fft(d.astype(np.longdouble), nf, 0)[:h], nk, 1), 1)
+    assert D.dtype == np.clongdouble
+    D = np.fft.ifft(np.fft.ifftshift(D * F.cone(h, nk, w), 1), nk, 1)
+    full = np.concatenate([D, np.conj(np.flipud(D[1:-1]))])
+    return np.real(np.fft.ifft(full, nf, 0))[:n1, :n2]
+
+
+@pytest.mark.parametrize("shape", [(129, 33), (1000, 300), (2500, 600), (6000, 200)])
+def test_error_against_long_double(fk, monkeypatch, shape):
+    """Root mean square error of the three kernels and of the library's
+    transforms against long double.  The four transforms have 2 log2(nf nk)
+    levels of additions, each rounding a value by at most half an ulp (2^-53)
+    in the mean square: the root of their number bounds the sum."""
+    d = np.random.default_rng(shape[0]).standard_normal(shape)
+    ref = _long_double(d, 0.05)
+    scale = np.sqrt(np.mean(ref.astype(np.float64) ** 2))
+
+    def err(x):
+        return float(np.sqrt(np.mean((x - ref) ** 2))) / scale
+
+    own = err(fk.fkdip(d, 0.05))
+    monkeypatch.setenv("SH_FK_1D", "1")
+    print(shape, "rms error: kernels", own, "library", err(fk.fkdip(d, 0.05)), flush=True)
+    assert own <= np.sqrt(2 * np.log2(F.nextpow2(shape[0]) * F.nextpow2(shape[1]))) * 2.0**-53
+
+
 def test_lengths_left_to_the_library(fk):
     """One step beyond the three kernels' range on each side."""
     for shape in [(64, 100), (16385, 40), (200, 32), (130, 4097)]:
