@@ -17,6 +17,7 @@
 // instructions a sample and wave), hidden by other blocks of the CU when
 // there are more than one.
 #include <algorithm>
+#include <type_traits>
 
 #include "predict.hpp"
 
@@ -80,17 +81,19 @@ __device__ inline __amdgpu_buffer_rsrc_t chain_rsrc(const void *p, unsigned long
 }
 
 // Row k of a plane of factor rows through a buffer resource: the lane's
-// offset in a register, the row's as the instruction's scalar offset, which
-// the resource's range check does not cover: rows past the last one are read
-// as the last one.
+// offset in a register, the row's as the instruction's scalar offset.  The
+// resource's range check does not cover that one, so a row past the last one
+// has to be asked for with END: it is read as the last one (512 x 256, eight
+// predictions: 519 us, 529 if every row is loaded so).
 template <int NB>
 struct ChainRows {
     __amdgpu_buffer_rsrc_t r;
     int lane;      // byte offset of the trace's row 0
     unsigned row;  // bytes from one sample to the next
     int last;      // the last row
+    template <bool END = false>
     __device__ void load(int k, float *o) const {
-        const int so = (int)__builtin_amdgcn_readfirstlane((unsigned)min(k, last) * row);
+        const int so = (int)__builtin_amdgcn_readfirstlane((unsigned)(END ? min(k, last) : k) * row);
         typedef float f2 __attribute__((ext_vector_type(2)));
         if constexpr (NB % 4 == 0) {
 #pragma unroll
@@ -121,7 +124,7 @@ __device__ inline void chain_forward(const ChainRows<NB> &F, float *y, int n1) {
 #pragma unroll
     for (int s = 0; s < D; s++) {
         if (s < D - NB) {
-            F.load(s, o[s]);
+            F.template load<true>(s, o[s]);
         } else {
 #pragma unroll
             for (int m = 0; m < NB; m++) o[s][m] = 0.0f;
@@ -133,7 +136,8 @@ __device__ inline void chain_forward(const ChainRows<NB> &F, float *y, int n1) {
     ch_f4 r[R];
 #pragma unroll
     for (int g = 0; g < R; g++) r[g] = reinterpret_cast<const ch_f4 *>(y)[g];
-    for (int k0 = 0; k0 < n1; k0 += D) {
+    auto group = [&](auto end, int k0) {
+        constexpr bool END = decltype(end)::value;  // the rows to come may lie past the last one
 #pragma unroll
         for (int g = 0; g < D / 4; g++) {
             ch_f4 v = r[g % R];
@@ -148,11 +152,14 @@ __device__ inline void chain_forward(const ChainRows<NB> &F, float *y, int n1) {
                 for (int m = NB - 1; m > 0; m--) b[m] = b[m - 1];
                 b[0] = t;
                 v[i] = t;
-                F.load(k0 + s + D - NB, o[(s + D - NB) % D]);
+                F.template load<END>(k0 + s + D - NB, o[(s + D - NB) % D]);
             }
             *reinterpret_cast<ch_f4 *>(y + k0 + 4 * g) = v;
         }
-    }
+    };
+    int k0 = 0;
+    for (; k0 + 2 * D - NB <= n1; k0 += D) group(std::false_type{}, k0);
+    for (; k0 < n1; k0 += D) group(std::true_type{}, k0);
 }
 
 // Backward substitution in place (banded_solve's second loop after the
@@ -164,7 +171,7 @@ __device__ inline void chain_backward(const ChainRows<NB> &F, float *y, int n1) 
     float o[D][NB], x[NB];
 #pragma unroll
     for (int s = 0; s < D; s++) {
-        F.load(top - D + s, o[s]);
+        F.template load<true>(top - D + s, o[s]);
 #pragma unroll
         for (int m = 0; m < NB; m++) o[s][m] = top - D + s < n1 ? o[s][m] : 0.0f;
     }
