@@ -80,20 +80,31 @@ __device__ inline __amdgpu_buffer_rsrc_t chain_rsrc(const void *p, unsigned long
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)(unsigned)bytes, 0x00020000);
 }
 
-// Row k of a plane of factor rows through a buffer resource: the lane's
-// offset in a register, the row's as the instruction's scalar offset.  The
-// resource's range check does not cover that one, so a row past the last one
-// has to be asked for with END: it is read as the last one (512 x 256, eight
-// predictions: 519 us, 529 if every row is loaded so).
+// Rows of a plane of factor rows through a buffer resource, one after the
+// other: the lane's offset in a register, the row's as the instruction's
+// scalar offset.  The resource's range check does not cover that one, so the
+// offset stops at the last row (or the first); a loop that stays below it
+// says so (END), for the two scalar instructions a row (512 x 256, eight
+// predictions: 525 us, 528 without).  The offset is hidden from the optimiser
+// after every step, which otherwise keeps those of a whole ring in scalar
+// registers and spills them (sint3d of 300 x 100 x 100 11.15 ms, 11.39
+// without).
 template <int NB>
 struct ChainRows {
     __amdgpu_buffer_rsrc_t r;
-    int lane;      // byte offset of the trace's row 0
-    unsigned row;  // bytes from one sample to the next
-    int last;      // the last row
-    template <bool END = false>
-    __device__ void load(int k, float *o) const {
-        const int so = (int)__builtin_amdgcn_readfirstlane((unsigned)(END ? min(k, last) : k) * row);
+    int lane;            // byte offset of the trace's row 0
+    unsigned row, last;  // bytes from one sample to the next; to the last one
+    template <bool END = true>
+    __device__ void up(unsigned &at) const {
+        at = __builtin_amdgcn_readfirstlane(END ? min(at + row, last) : at + row);
+        asm volatile("" : "+s"(at));
+    }
+    __device__ void down(unsigned &at) const {
+        at = __builtin_amdgcn_readfirstlane(at - min(at, row));
+        asm volatile("" : "+s"(at));
+    }
+    __device__ void load(unsigned at, float *o) const {
+        const int so = (int)__builtin_amdgcn_readfirstlane(at);
         typedef float f2 __attribute__((ext_vector_type(2)));
         if constexpr (NB % 4 == 0) {
 #pragma unroll
@@ -121,10 +132,12 @@ struct ChainRows {
 template <int NB, int D>
 __device__ inline void chain_forward(const ChainRows<NB> &F, float *y, int n1) {
     float o[D][NB], b[NB];
+    unsigned at = 0;
 #pragma unroll
     for (int s = 0; s < D; s++) {
         if (s < D - NB) {
-            F.template load<true>(s, o[s]);
+            F.load(at, o[s]);
+            F.up(at);
         } else {
 #pragma unroll
             for (int m = 0; m < NB; m++) o[s][m] = 0.0f;
@@ -137,7 +150,7 @@ __device__ inline void chain_forward(const ChainRows<NB> &F, float *y, int n1) {
 #pragma unroll
     for (int g = 0; g < R; g++) r[g] = reinterpret_cast<const ch_f4 *>(y)[g];
     auto group = [&](auto end, int k0) {
-        constexpr bool END = decltype(end)::value;  // the rows to come may lie past the last one
+        constexpr bool END = decltype(end)::value;  // the rows to come reach the last one
 #pragma unroll
         for (int g = 0; g < D / 4; g++) {
             ch_f4 v = r[g % R];
@@ -152,29 +165,34 @@ __device__ inline void chain_forward(const ChainRows<NB> &F, float *y, int n1) {
                 for (int m = NB - 1; m > 0; m--) b[m] = b[m - 1];
                 b[0] = t;
                 v[i] = t;
-                F.template load<END>(k0 + s + D - NB, o[(s + D - NB) % D]);
+                F.load(at, o[(s + D - NB) % D]);  // row k0 + s + D - NB
+                F.template up<END>(at);
             }
             *reinterpret_cast<ch_f4 *>(y + k0 + 4 * g) = v;
         }
     };
     int k0 = 0;
-    for (; k0 + 2 * D - NB <= n1; k0 += D) group(std::false_type{}, k0);
+    for (; k0 + 2 * D - NB < n1; k0 += D) group(std::false_type{}, k0);
     for (; k0 < n1; k0 += D) group(std::true_type{}, k0);
 }
 
 // Backward substitution in place (banded_solve's second loop after the
 // division): y[k] -= o_m[k] y[k+1+m], from the end of the padding (zeros
-// there, and its factor rows are taken as zeros: its values stay zero).
+// there, and the last row's entries, which its rows are read as, are zeros,
+// since no sample lies beyond: its values stay zero).
 template <int NB, int D>
 __device__ inline void chain_backward(const ChainRows<NB> &F, float *y, int n1) {
     const int top = (n1 + D - 1) / D * D;
     float o[D][NB], x[NB];
+    const unsigned start = (unsigned)(top - D) * F.row;
+    unsigned at = start;
 #pragma unroll
     for (int s = 0; s < D; s++) {
-        F.template load<true>(top - D + s, o[s]);
-#pragma unroll
-        for (int m = 0; m < NB; m++) o[s][m] = top - D + s < n1 ? o[s][m] : 0.0f;
+        F.load(at, o[s]);
+        F.up(at);
     }
+    at = start;
+    F.down(at);
 #pragma unroll
     for (int m = 0; m < NB; m++) x[m] = 0.0f;
     constexpr int R = 2;
@@ -196,7 +214,8 @@ __device__ inline void chain_backward(const ChainRows<NB> &F, float *y, int n1) 
                 for (int m = NB - 1; m > 0; m--) x[m] = x[m - 1];
                 x[0] = t;
                 v[i] = t;
-                F.load(max(k0 + s - D, 0), o[s]);
+                F.load(at, o[s]);  // row k0 + s - D
+                F.down(at);
             }
             *reinterpret_cast<ch_f4 *>(y + k0 + 4 * g) = v;
         }
@@ -312,7 +331,7 @@ __device__ inline void chain_solve(const ChainBlock &B, float *row, const float 
     const float *fo = Fv + (long)NB * B.base, *fd = Fv + (long)NB * n + B.base;
     const bool walker = threadIdx.x < (unsigned)B.nt && act;
     const ChainRows<NB> F{chain_rsrc(fo, (unsigned long)B.slice * NB * 4), ip * NB * 4, (unsigned)B.n2 * NB * 4,
-                          B.n1 - 1};
+                          (unsigned)(B.n1 - 1) * (unsigned)B.n2 * NB * 4};
     __syncthreads();
     if (walker) {
         __builtin_amdgcn_s_setprio(3);
