@@ -83,12 +83,12 @@ __device__ inline __amdgpu_buffer_rsrc_t chain_rsrc(const void *p, unsigned long
 // Rows of a plane of factor rows through a buffer resource, one after the
 // other: the lane's offset in a register, the row's as the instruction's
 // scalar offset.  The resource's range check does not cover that one, so the
-// offset stops at the last row (or the first); a loop that stays below it
-// says so (END), for the two scalar instructions a row (512 x 256, eight
-// predictions: 525 us, 528 without).  The offset is hidden from the optimiser
-// after every step, which otherwise keeps those of a whole ring in scalar
-// registers and spills them (sint3d of 300 x 100 x 100 11.15 ms, 11.39
-// without).
+// offset stops at the last row, in the loops that reach it (END), and at the
+// first one by a step of zero (a scalar instruction a row each; with both in
+// every row 512 x 256, eight predictions, takes 528 us, so 500).  The offset
+// is hidden from the optimiser after every step, which otherwise keeps those
+// of a whole ring in scalar registers and spills them (sint3d of 300 x 100 x
+// 100 11.15 ms, 11.39 without).
 template <int NB>
 struct ChainRows {
     __amdgpu_buffer_rsrc_t r;
@@ -99,8 +99,8 @@ struct ChainRows {
         at = __builtin_amdgcn_readfirstlane(END ? min(at + row, last) : at + row);
         asm volatile("" : "+s"(at));
     }
-    __device__ void down(unsigned &at) const {
-        at = __builtin_amdgcn_readfirstlane(at - min(at, row));
+    static __device__ void down(unsigned &at, unsigned step) {
+        at = __builtin_amdgcn_readfirstlane(at - step);
         asm volatile("" : "+s"(at));
     }
     __device__ void load(unsigned at, float *o) const {
@@ -192,7 +192,6 @@ __device__ inline void chain_backward(const ChainRows<NB> &F, float *y, int n1) 
         F.up(at);
     }
     at = start;
-    F.down(at);
 #pragma unroll
     for (int m = 0; m < NB; m++) x[m] = 0.0f;
     constexpr int R = 2;
@@ -200,6 +199,7 @@ __device__ inline void chain_backward(const ChainRows<NB> &F, float *y, int n1) 
 #pragma unroll
     for (int g = 0; g < R; g++) r[g] = *reinterpret_cast<const ch_f4 *>(y + top - 4 * R + 4 * g);
     for (int k0 = top - D; k0 >= 0; k0 -= D) {
+        const unsigned step = k0 ? F.row : 0;  // the first group has no rows before it
 #pragma unroll
         for (int g = D / 4 - 1; g >= 0; g--) {
             ch_f4 v = r[g % R];
@@ -214,8 +214,8 @@ __device__ inline void chain_backward(const ChainRows<NB> &F, float *y, int n1) 
                 for (int m = NB - 1; m > 0; m--) x[m] = x[m - 1];
                 x[0] = t;
                 v[i] = t;
+                F.down(at, step);
                 F.load(at, o[s]);  // row k0 + s - D
-                F.down(at);
             }
             *reinterpret_cast<ch_f4 *>(y + k0 + 4 * g) = v;
         }
