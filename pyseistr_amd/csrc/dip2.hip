@@ -9,9 +9,11 @@
 // the smoothed gradient and the conjugate directions with its neighbours.
 // The float operations on a sample and their order are those of the launches
 // (dip.hip), so the dips are the same; only the double sums are added in
-// another order.  512 x 256, 5 x 20 iterations: 2750 -> 805 us; 128 x 64 about
-// 2000 -> 440 us.  What bounds it: about 100 phases of 5-8 us, each a round
-// trip of the exchange, a barrier and the two stencils.  (A batch of sections
+// another order.  512 x 256, 5 x 20 iterations: 2800 -> 920 us (the kernel 775 in
+// another run); 128 x 64: the kernel 390 us of about 2000 before.  What bounds
+// it: dependent phases, each a round trip of the exchange, a barrier and the
+// two stencils: two a CG iteration and two or three a Gauss-Newton step, 217 at
+// most.  (A batch of sections
 // as teams of blocks in one launch ran no faster than its launches: with the
 // chip full both are bound by the work in the tiles.)
 //

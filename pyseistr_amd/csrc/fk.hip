@@ -106,8 +106,8 @@ __global__ void fk_crop1(const double2 *__restrict__ C, double *__restrict__ out
 // each) fourteen times.  6000 x 2500 (8192 x 4096 padded): 1116 us before,
 // now 86 (rows), 150 (space) and 70 (rows back), where the copy's rate takes
 // 60, 70 and 60.  Error against long double, root mean square, over 129 x 33
-// to 6000 x 2500: 2.4e-16 to 4.0e-16 (the library's transforms: 3.5e-16 to
-// 6.7e-16).
+// to 6000 x 200: 2.2e-16 to 3.7e-16 (the library's transforms: 4.0e-16 to
+// 5.7e-16).
 // ---------------------------------------------------------------------------
 __device__ inline long spec_at(int f, long c, long n2) { return ((f >> 3) * n2 + c) * 8 + (f & 7); }
 

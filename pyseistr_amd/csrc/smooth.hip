@@ -259,7 +259,8 @@ smoothc_resident(const float *in, float *out, int n1, int n2, int n3, int ax, in
 
 // Lines a block holds, 0 if they do not fit (the kernels above take long
 // lines, and radii beyond the axis in the adj = 0 form, whose overhangs then
-// fold more than once).  At least three blocks a CU, at least four lines.
+// fold more than once).  At least four lines; three blocks a CU where 32 lines
+// or more fit so, two with fewer.
 int resident_lines(int nx, int nb, bool adj) {
     if (nx > 1 << 16 || nb > 1 << 16 || (!adj && nb > nx)) return 0;
     const long np = nx + 2L * nb;
