@@ -1019,12 +1019,11 @@ bool spray2_blocks(const Pwsmooth2 &P) {
 // Factor cache of P into caller-provided buffers: scr holds 2*nthr*n1
 // floats (solver scratch, then the running trace planes), F
 // 3 * fac_plane_floats(2 * order, n): the two factor variants, then the
-// filter taps of the slopes (which the block kernels form themselves).
+// filter taps of the slopes.  The block kernels, which form the taps
+// themselves, leave scr (it may be null) and the third plane alone.
 int pws2_prepare_bufs(sh_ctx *ctx, Pwsmooth2 &P, float *scr, float *F) {
     long n = (long)P.n1 * P.n2 * P.n3;
     P.nthr = pws2_nthr(P.n2, P.n3);
-    P.scr = scr;
-    P.tr = P.scr + (long)P.nthr * P.n1;
     P.F = F;
     if (spray2_blocks(P)) {
         PROF_A(ctx);
@@ -1032,6 +1031,8 @@ int pws2_prepare_bufs(sh_ctx *ctx, Pwsmooth2 &P, float *scr, float *F) {
         PROF_B(ctx, "chain2_rows+ldl", 4.0 * (double)n);
         return SH_OK;
     }
+    P.scr = scr;
+    P.tr = P.scr + (long)P.nthr * P.n1;
     const int TB2 = spray2_tb();
     dim3 grid(ceil_div(2L * P.n2, TB2), P.n3);
     PROF_A(ctx);
@@ -1049,9 +1050,12 @@ int pws2_prepare_bufs(sh_ctx *ctx, Pwsmooth2 &P, float *scr, float *F) {
 int pws2_prepare(sh_ctx *ctx, Pwsmooth2 &P, int slot_scr, int slot_F) {
     long n = (long)P.n1 * P.n2 * P.n3;
     const long nthr = pws2_nthr(P.n2, P.n3);
+    // the block kernels need neither the scratch nor the taps' plane
+    const bool blocks = spray2_blocks(P);
     float *scr = nullptr, *F = nullptr;
-    SH_TRY(sh_slot(ctx, slot_scr, (size_t)nthr * P.n1 * 2 * sizeof(float), (void **)&scr));
-    SH_TRY(sh_slot(ctx, slot_F, (size_t)3 * fac_plane_floats(2 * P.order, n) * sizeof(float), (void **)&F));
+    if (!blocks) SH_TRY(sh_slot(ctx, slot_scr, (size_t)nthr * P.n1 * 2 * sizeof(float), (void **)&scr));
+    SH_TRY(sh_slot(ctx, slot_F, (size_t)(blocks ? 2 : 3) * fac_plane_floats(2 * P.order, n) * sizeof(float),
+                   (void **)&F));
     return pws2_prepare_bufs(ctx, P, scr, F);
 }
 
